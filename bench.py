@@ -256,13 +256,13 @@ def measure_kernels(model_cfg, iters, only=None):
             us = time_launches(lambda s: fk.relative_bias(q0, k0, pkh, pqh, c2p, p2c, km, scale, B, H, L, D, P), [0],
                                iters)
             nbytes = 2 * B * H * L * D * 2 + common + B * H * L * L * 2
-            out["general_relative_bias"] = dict(kernel="general_mfma_kernel<false>", shape=[B, H, L, L], us=us,
+            out["general_relative_bias"] = dict(kernel="relative_bias_mfma_kernel", shape=[B, H, L, L], us=us,
                                                 bytes=nbytes, gbs=nbytes / us / 1e3, bound="hbm", launches_per_step=0)
         if want("general_fused_attention"):
             us = time_launches(lambda s: fk.fused_attention(q0, k0, v0, pkh, pqh, c2p, p2c, km, scale, B, H, L, D, P),
                                [0], iters)
             nbytes = 3 * B * H * L * D * 2 + common + B * L * H * D * 2
-            out["general_fused_attention"] = dict(kernel="general_mfma_kernel<true>", shape=[B, H, L, D], us=us,
+            out["general_fused_attention"] = dict(kernel="fused_attention_mfma_kernel", shape=[B, H, L, D], us=us,
                                                   bytes=nbytes, gbs=nbytes / us / 1e3, bound="hbm",
                                                   launches_per_step=0)
         del c2p, p2c, q0, k0, v0

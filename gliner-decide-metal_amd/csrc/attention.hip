@@ -7,9 +7,11 @@
 // back the FusedKernels-shaped entry points.  The encoder itself runs the
 // staged kernel of deberta_attention.hip, which derives the indices from the
 // bucket function directly.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <initializer_list>
+#include <type_traits>
 
 #include "gd_common.hpp"
 #include "gd_kernels.hpp"
@@ -113,62 +115,411 @@ __global__ __launch_bounds__(64) void fused_attention_general_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// The general-index kernels on the matrix cores (D = 64, L a multiple of 16,
-// L <= 512, P <= 65536).  A workgroup of 4 waves owns (b, h, 64 queries),
-// wave w queries q0 + 16 w .. + 15, and takes the keys in blocks of 64: the
-// relative bias gives each key block a workgroup of its own, the fused
-// attention walks all of them.  25 KB of LDS per workgroup; the bias kernel's
-// 86 VGPRs let five workgroups share a CU, the fused kernel's 127 (it also
-// carries the softmax state and the output) four.  Time follows occupancy:
-// the passes below are chains of LDS round trips and barriers.
-// For a key block, every pass over 64 positions of the tables computes
-// C2P = Q . posK[pass]^T (v_mfma_f32_16x16x32_f16, fp32) into an LDS table
-// [query][position], or per 16-key block P2C = K . posQ[pass]^T into a table
-// [key][position]; each score takes its two terms from the tables at its
-// indices when they fall in the pass.  The c2p passes run before the p2c
-// passes, so a score accumulates (x + c2p) + p2c, x = -0 for the bias and
-// x = q.k for the fused attention: the reference's fp32 sum, term by term,
-// whatever pass a term came from.  Indices outside [0, P) are clamped, as the
-// per-query kernels do.
+// The relative bias with index tensors on the matrix cores (D = 64, L <= 512,
+// any length, P <= 65536).  A workgroup of 4 waves owns 64 queries x 64 keys
+// of one head and walks `nb` batch rows: the index tensors and the position
+// tables do not depend on the batch row, so a wave reads its indices and its
+// table rows once, keeps the rows as MFMA fragments and the scores' table
+// offsets in registers, and per batch row brings only Q and K.
 //
-// Fused attention: scores (x + c2p + p2c) * scale (masked keys -65504) feed
-// an online softmax per query row (running max seeded at -65504, the
-// reference's seed), and P . V runs on the matrix cores with P split into
-// fp16 hi + lo (V rows in LDS, read transposed by ds_read_b64_tr_b16); the
-// output row is divided by the row's sum at the end.
+// Relative-position indices of 16 x 64 positions span at most 79 rows, so
+// from exactly the least index on five 16-row tiles of posK serve the c2p
+// terms of a wave's 16 queries, and five of posQ the p2c terms of its 16 keys:
+// C2P = Q . posK^T and P2C = K . posQ^T (v_mfma_f32_16x16x32_f16, fp32) go
+// through LDS tables of 80 columns, and each score takes one term from each at
+// its index.  C2P rows are read by the wave that writes them; P2C rows by all
+// four, so they alternate between two tables with one barrier per batch row.
+// Wider spans (arbitrary index tensors) run further windows over the same
+// tables, a position outside the window at hand reading a -0 column.  A score
+// is (-0 + c2p) + p2c, term by term the reference's fp32 sum.  Indices outside
+// [0, P) are clamped, as the per-query kernel does.  Queries and keys past L
+// repeat the last one (indices of a valid pair of the tile); their scores are
+// not stored.
+//
+// Bound by the batch row's chain (MFMA, table, gather, barrier, store) with
+// two waves per SIMD (230-247 VGPRs).  B = 32, H = 16, L = 256: 36.4 us
+// against 72.5 us of a kernel that read indices and table rows for every batch
+// row and ran 64-row windows of either table, a gather per window; at 5 TB/s
+// its 111 MB take 22 us.
 // ---------------------------------------------------------------------------
-constexpr int kGenPass = 64;               // table positions per pass
-constexpr int kGenStride = kGenPass + 4;   // fp32 row stride: float4 stores of 8 lanes hit 32 distinct banks
-// Column kGenPass of every table row holds -0, the term of a position outside
-// the pass (x + -0 = x for every fp32 x, signed zeros included).
-__device__ __forceinline__ int gen_col(int c) { return (unsigned)c < (unsigned)kGenPass ? c : kGenPass; }
-constexpr int kGenKeyBlocks = 4;           // 16-key blocks per key block (64 keys)
-// The table-rows buffer also holds the fused kernel's K rows and V rows of a key block.
-static_assert(16 * kGenKeyBlocks == kGenPass, "a key block's K / V rows fill the table-rows buffer");
+constexpr int64_t kGenCus = 256;  // compute units of the device the grids are sized for
+constexpr int kGenKeyBlocks = 4;  // 16-key blocks per key block (64 keys)
+constexpr int kBiasTiles = 5;     // 16-row tiles of a table window
+constexpr int kBiasCols = 16 * kBiasTiles;
+// fp32 row stride of the tables: float4 stores of 8 consecutive rows hit 32
+// distinct banks; column kBiasCols holds the -0 of a position outside the window.
+constexpr int kBiasStride = kBiasCols + 4;
 
-typedef __attribute__((address_space(3))) void gen_lds_void_t;
+// Least of a wave's values (VALU moves, no LDS round trips).
+template <int CTRL>
+__device__ __forceinline__ int gen_dpp(int v) { return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false); }
+__device__ __forceinline__ int gen_wave_min(int v) {
+  v = min(v, gen_dpp<0xB1>(v));   // quad_perm [1,0,3,2]
+  v = min(v, gen_dpp<0x4E>(v));   // quad_perm [2,3,0,1]
+  v = min(v, gen_dpp<0x141>(v));  // row_half_mirror
+  v = min(v, gen_dpp<0x140>(v));  // row_mirror
+  return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+             min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// Workgroups per CU of the form for one batch row (four would spill: B = 1, L =
+// 512 takes 18.3 us with three, 24.4 us with four).
+constexpr int kBiasOneWaves = 3;
+
+// W: the largest of 8, 4, 2 and 1 that divides L, the halfs of the output
+// pieces (every row starts aligned to one); from 4 on the c2p indices and the
+// mask of four consecutive keys are one aligned load.  MULTI: the workgroup
+// walks several batch rows.  With one there is nothing to keep: P2C takes the
+// C2P rows' place, and kBiasOneWaves workgroups share a CU.
+template <int W, bool MULTI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 : kBiasOneWaves, MULTI ? 2 : kBiasOneWaves))) void relative_bias_mfma_kernel(
+    const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ pos_key,
+    const half_t* __restrict__ pos_query, const int32_t* __restrict__ c2p_idx, const int32_t* __restrict__ p2c_idx,
+    const half_t* __restrict__ key_mask, float scale, int B, int H, int L, int P, int nb, half_t* __restrict__ out) {
+  constexpr int KB = kGenKeyBlocks;
+  constexpr bool VEC = W >= 4;
+  __shared__ __attribute__((aligned(16))) float ctab[64 * kBiasStride];     // C2P [query][column]
+  __shared__ __attribute__((aligned(16))) float ptabs[MULTI ? 2 : 1][MULTI ? 64 * kBiasStride : 4];  // P2C [key][column]
+  auto ptab = [&](int i) -> float* { return MULTI ? ptabs[i] : ctab; };
+  __shared__ int ranges[4][2 + 2 * KB];  // per wave: least c2p, -c2p, then p2c and -p2c of each 16-key block
+  // Workgroup -> (h, 64-query block qb, key block ky, batch rows b0 ..).
+  // Workgroups go to the 8 XCDs round-robin; with H a multiple of 8, XCD x
+  // takes heads x H / 8 .. (x + 1) H / 8 - 1 only, so its L2 holds just those
+  // heads' index tensors and position tables.
+  const int nq = (L + 63) / 64;
+  int h, qb, ky, b0;
+  {
+    const int w = blockIdx.x;
+    int r;
+    if (H % 8 == 0) {
+      const int hx = H / 8, l = w >> 3;
+      h = (w & 7) * hx + l % hx;
+      r = l / hx;
+    } else {
+      h = w % H;
+      r = w / H;
+    }
+    qb = r % nq;
+    r /= nq;
+    ky = r % nq;
+    b0 = r / nq * nb;
+  }
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lc = lane & 15, g = lane >> 4;
+  const int qw = qb * 64 + 16 * wave;            // the wave's first query
+  const int qr = qw + lc < L ? qw + lc : L - 1;  // this lane's query (keys 4 g .. 4 g + 3 of a block)
+  const int kw = 64 * ky + 16 * wave + lc;       // this lane's key of the wave's P2C rows
+  const int kr = kw < L ? kw : L - 1;
+  // A wave with neither a query nor a P2C key ends here: the barriers below
+  // wait for the waves that go on, and nothing reads this one's rows.
+  if (qw >= L && 64 * ky + 16 * wave >= L) return;
+  const half_t* pkh = pos_key + (int64_t)h * P * 64;
+  const half_t* pqh = pos_query + (int64_t)h * P * 64;
+  const int32_t* c2ph = c2p_idx + (int64_t)h * L * L;
+  const int32_t* p2ch = p2c_idx + (int64_t)h * L * L;
+  auto clampi = [&](int x) { return x < 0 ? 0 : (x >= P ? P - 1 : x); };
+  auto key_of = [&](int kb) { return 64 * ky + 16 * kb + 4 * g; };  // this lane's first key of block kb
+  auto row_frags = [&](const half_t* base, int row, half8_t (&f)[2]) {
+    f[0] = *reinterpret_cast<const half8_t*>(base + (uint32_t)(row * 64 + 8 * g));
+    f[1] = *reinterpret_cast<const half8_t*>(base + (uint32_t)(row * 64 + 32 + 8 * g));
+  };
+  // Of one batch row: fragments of this wave's queries and of its P2C keys,
+  // the mask of this lane's keys.
+  struct Row {
+    half8_t q[2], k[2];
+    half4_t mask[KB];
+  };
+  auto fetch = [&](int b, Row& x) {
+    const int64_t bh = (int64_t)b * H + h;
+    row_frags(q + bh * L * 64, qr, x.q);
+    row_frags(k + bh * L * 64, kr, x.k);
+    const half_t* mrow = key_mask + (int64_t)b * L;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const int key = key_of(kb);
+      if constexpr (VEC) {
+        x.mask[kb] = *reinterpret_cast<const half4_t*>(mrow + (uint32_t)(key < L ? key : L - 4));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x.mask[kb][j] = mrow[(uint32_t)(key + j < L ? key + j : L - 1)];
+      }
+    }
+  };
+
+  // ---- once: indices, their ranges, table rows ----
+  int ci[KB][4], pi[KB][4];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int key = key_of(kb);
+    if constexpr (VEC) {
+      const int kc = key < L ? key : L - 4;
+      const int4 x = *reinterpret_cast<const int4*>(c2ph + (uint32_t)(qr * L + kc));
+      ci[kb][0] = x.x, ci[kb][1] = x.y, ci[kb][2] = x.z, ci[kb][3] = x.w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pi[kb][j] = p2ch[(uint32_t)((kc + j) * L + qr)];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int kc = key + j < L ? key + j : L - 1;
+        ci[kb][j] = c2ph[(uint32_t)(qr * L + kc)];
+        pi[kb][j] = p2ch[(uint32_t)(kc * L + qr)];
+      }
+    }
+  }
+  // Fragments of the 16-row tile of a table from row `row0` on (rows past P
+  // repeat row P - 1).
+  auto tile_frags = [&](const half_t* table, int row0, half8_t (&f)[2]) {
+    row_frags(table, row0 + lc < P ? row0 + lc : P - 1, f);
+  };
+  half8_t ct[kBiasTiles][2], pt[kBiasTiles][2];
+  uint32_t cp[KB][4];  // the clamped indices, c2p | p2c << 16
+  auto c_of = [](uint32_t x) { return (int)(x & 0xFFFFu); };
+  auto p_of = [](uint32_t x) { return (int)(x >> 16); };
+  Row cur, nxt;
+  fetch(b0, nxt);
+  {
+    int c_mn = P, c_mx = 0, p_mn[KB], p_mx[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      p_mn[kb] = P, p_mx[kb] = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        ci[kb][j] = clampi(ci[kb][j]), pi[kb][j] = clampi(pi[kb][j]);
+        c_mn = min(c_mn, ci[kb][j]), c_mx = max(c_mx, ci[kb][j]);
+        p_mn[kb] = min(p_mn[kb], pi[kb][j]), p_mx[kb] = max(p_mx[kb], pi[kb][j]);
+        cp[kb][j] = (uint32_t)ci[kb][j] | ((uint32_t)pi[kb][j] << 16);
+      }
+    }
+    int r[2 + 2 * KB];
+    r[0] = gen_wave_min(c_mn), r[1] = gen_wave_min(-c_mx);
+    // the c2p rows need no other wave's range: in flight from here
+#pragma unroll
+    for (int tp = 0; tp < kBiasTiles; ++tp) tile_frags(pkh, r[0] + 16 * tp, ct[tp]);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) r[2 + 2 * kb] = gen_wave_min(p_mn[kb]), r[3 + 2 * kb] = gen_wave_min(-p_mx[kb]);
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < 2 + 2 * KB; ++i) ranges[wave][i] = r[i];
+    }
+  }
+  stage_barrier();
+  // least index of the wave's c2p and of each block's p2c, greatest spans
+  int c_lo = 0;
+  int p_lo[KB], c_end = 0, p_all = P, p_end = 0;
+  bool narrow = true;  // uniform over the workgroup: every window is one
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (64 * qb + 16 * w >= L && w != wave) continue;  // no query: its indices are another wave's
+    const int lo = __builtin_amdgcn_readfirstlane(ranges[w][0]), hi = -__builtin_amdgcn_readfirstlane(ranges[w][1]);
+    narrow = narrow && hi - lo < kBiasCols;
+    if (w == wave) c_lo = lo, c_end = hi;
+  }
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    int lo = P, hi = P;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (64 * qb + 16 * w >= L) continue;
+      lo = min(lo, ranges[w][2 + 2 * kb]), hi = min(hi, ranges[w][3 + 2 * kb]);
+    }
+    p_lo[kb] = __builtin_amdgcn_readfirstlane(lo);
+    hi = -__builtin_amdgcn_readfirstlane(hi);
+    narrow = narrow && hi - p_lo[kb] < kBiasCols;
+    p_all = min(p_all, p_lo[kb]), p_end = max(p_end, hi);
+  }
+  // One tile's products into a table row's columns.
+  auto product = [&](const half8_t (&a)[2], const half8_t (&f)[2], float* row, int tp) {
+    float4_t r = {0.f, 0.f, 0.f, 0.f};
+    r = mfma16x16x32(a[0], f[0], r);
+    r = mfma16x16x32(a[1], f[1], r);  // lane: row lc, columns 16 tp + 4 g + i
+    *reinterpret_cast<float4_t*>(row + 16 * tp + 4 * g) = r;
+  };
+  float* const crow = ctab + (16 * wave + lc) * kBiasStride;
+  const int b_end = !MULTI ? b0 + 1 : (b0 + nb < B ? b0 + nb : B);
+
+  // ---- scores: (c2p + p2c) * scale, masked keys -65504, staged through the
+  // wave's C2P rows into row pieces of up to 128 bytes ----
+  auto finish = [&](int b, const float (&acc)[KB][4], const half4_t (&mask)[KB]) {
+    half_t* const stage = reinterpret_cast<half_t*>(ctab + 16 * wave * kBiasStride);
+    wave_lds_sync();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      half4_t sv;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        sv[j] = (float)mask[kb][j] < -60000.f ? (half_t)-65504.f : (half_t)(acc[kb][j] * scale);
+      *reinterpret_cast<half4_t*>(stage + lc * (2 * kBiasStride) + 16 * kb + 4 * g) = sv;
+    }
+    wave_lds_sync();
+    typedef _Float16 piece_t __attribute__((ext_vector_type(W)));
+    constexpr int PER = 16 * KB / W, ROWS = 64 / PER;  // pieces per row, rows per store
+    const int r = lane / PER, cc = lane % PER * W;
+    const uint32_t off = (uint32_t)(r * L + 64 * ky + cc);
+    half_t* const orow = out + (((int64_t)b * H + h) * L + qw) * L;  // uniform
+    // (the next batch row's loads are waited for here: behind the stores, the
+    // wait would be for the stores too)
+    if constexpr (MULTI) {
+      asm volatile("" : "+v"(nxt.q[0]), "+v"(nxt.q[1]), "+v"(nxt.k[0]), "+v"(nxt.k[1]));
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(nxt.mask[kb]));
+    }
+#pragma unroll
+    for (int r0 = 0; r0 < 16; r0 += ROWS)
+      if (qw + r0 + r < L && 64 * ky + cc < L)
+        *reinterpret_cast<piece_t*>(orow + (int64_t)r0 * L + off) =
+            *reinterpret_cast<const piece_t*>(stage + (r0 + r) * (2 * kBiasStride) + cc);
+    wave_lds_sync();
+  };
+
+  if (narrow) {
+    int p_own = p_lo[0];
+#pragma unroll
+    for (int kb = 1; kb < KB; ++kb) p_own = wave == kb ? p_lo[kb] : p_own;
+#pragma unroll
+    for (int tp = 0; tp < kBiasTiles; ++tp) tile_frags(pqh, p_own + 16 * tp, pt[tp]);
+    // (used here, so that they are waited for here: a wait inside the loop
+    // would also wait for the next batch row's loads, issued after them)
+#pragma unroll
+    for (int tp = 0; MULTI && tp < kBiasTiles; ++tp)
+      asm volatile("" : "+v"(ct[tp][0]), "+v"(ct[tp][1]), "+v"(pt[tp][0]), "+v"(pt[tp][1]));
+    int pbuf = 0;
+    for (int b = b0; b < b_end; ++b) {  // uniform
+      cur = nxt;
+      if (b + 1 < b_end) fetch(b + 1, nxt);
+      float* const pt_b = ptab(pbuf);
+      float* const prow = pt_b + (16 * wave + lc) * kBiasStride;
+#pragma unroll
+      for (int tp = 0; tp < kBiasTiles; ++tp) product(ct[tp], cur.q, crow, tp);
+      if constexpr (MULTI) {
+#pragma unroll
+        for (int tp = 0; tp < kBiasTiles; ++tp) product(pt[tp], cur.k, prow, tp);
+      }
+      wave_lds_sync();
+      float acc[KB][4];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[kb][j] = crow[c_of(cp[kb][j]) - c_lo];
+      if constexpr (!MULTI) {
+        wave_lds_sync();
+#pragma unroll
+        for (int tp = 0; tp < kBiasTiles; ++tp) product(pt[tp], cur.k, prow, tp);
+      }
+      stage_barrier();  // P2C rows visible; the last batch row's P2C reads are a barrier back
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[kb][j] += pt_b[(16 * kb + 4 * g + j) * kBiasStride + (p_of(cp[kb][j]) - p_lo[kb])];
+      if constexpr (!MULTI) stage_barrier();  // the scores are staged in the rows that were read
+      finish(b, acc, cur.mask);
+      pbuf ^= 1;
+    }
+  } else {
+    for (int b = b0; b < b_end; ++b) {  // uniform
+      cur = nxt;
+      if (b + 1 < b_end) fetch(b + 1, nxt);
+      // (the windows' addresses stay inside the loop: hoisting them all would
+      // spill registers)
+      int base = 0;
+      asm volatile("" : "+v"(base));
+      base = __builtin_amdgcn_readfirstlane(base);
+      int lo = c_lo + base, plo = p_all + base;
+      float acc[KB][4];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[kb][j] = -0.0f;
+      if (lane < 16) crow[kBiasCols] = -0.0f;
+      for (; lo <= c_end; lo += kBiasCols) {  // uniform within the wave
+#pragma unroll
+        for (int tp = 0; tp < kBiasTiles; ++tp) {
+          half8_t f[2];
+          tile_frags(pkh, lo + 16 * tp, f);
+          product(f, cur.q, crow, tp);
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[kb][j] += crow[min((uint32_t)(c_of(cp[kb][j]) - lo), (uint32_t)kBiasCols)];
+        wave_lds_sync();
+      }
+      float* const prow = ptab(0) + (16 * wave + lc) * kBiasStride;
+      if (lane < 16) prow[kBiasCols] = -0.0f;
+      for (; plo <= p_end; plo += kBiasCols) {  // uniform over the workgroup
+#pragma unroll
+        for (int tp = 0; tp < kBiasTiles; ++tp) {
+          half8_t f[2];
+          tile_frags(pqh, plo + 16 * tp, f);
+          product(f, cur.k, prow, tp);
+        }
+        stage_barrier();
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[kb][j] += ptab(0)[(16 * kb + 4 * g + j) * kBiasStride + min((uint32_t)(p_of(cp[kb][j]) - plo), (uint32_t)kBiasCols)];
+        stage_barrier();
+      }
+      finish(b, acc, cur.mask);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The fused attention with index tensors on the matrix cores (D = 64, L <=
+// 512, any length, P <= 65536).  A workgroup of 4 waves owns (b, h, 64
+// queries), wave w queries q0 + 16 w .. + 15, and walks the keys in blocks of
+// 64.  C2P and P2C go through an LDS table of 80 columns from the least index
+// of the wave's 16 x 64 positions on, as in the bias kernel; here each key
+// block needs fresh table rows, so a window of 128 rows of each table (the 64 x
+// 64 tile's relative positions span at most 127) comes by DMA for all four
+// waves.  Wider spans run further windows.  Every c2p window precedes every p2c
+// window, so a score accumulates (q.k + c2p) + p2c, the reference's fp32 sum,
+// term by term.
+//
+// Scores (masked keys -65504, keys past L -inf) feed an online softmax per
+// query row (running max seeded at -65504, the reference's seed), and P . V
+// runs on the matrix cores with P split into fp16 hi + lo (V rows in LDS, read
+// transposed by ds_read_b64_tr_b16); the output row is divided by the row's
+// sum at the end.  The next key block's windows, K and V rows come by DMA during
+// the softmax and P . V, its indices a block earlier; two barriers per block.
+// Bound by the block's chain of LDS round trips with two waves per SIMD (79 KB
+// of LDS, 240 VGPRs).  B = 8, H = 16, L = 200: 24.8 us (the per-query kernel,
+// which served every length that is no multiple of 16, 495 us); B = 32, L =
+// 256: 88 us (64-row windows, a gather per window: 97 us).
+// ---------------------------------------------------------------------------
+constexpr int kGenWin = 128;  // table rows per window
+
 typedef __attribute__((address_space(3))) half_t gen_lds_half_t;
 typedef short gen_short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) gen_short4_t gen_lds_short4_t;
 
+// A row of zeros: the V rows of keys past L.
+__device__ __attribute__((aligned(16))) const half_t g_zero_row[64] = {};
+
 __device__ __forceinline__ int gen_swz(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
-template <bool FUSED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FUSED ? 4 : 5, FUSED ? 4 : 5))) void general_mfma_kernel(
+// VEC: L is a multiple of 4, so the c2p indices and the mask of four
+// consecutive keys are one aligned load.
+template <bool VEC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void fused_attention_mfma_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     const half_t* __restrict__ pos_key, const half_t* __restrict__ pos_query, const int32_t* __restrict__ c2p_idx,
     const int32_t* __restrict__ p2c_idx, const half_t* __restrict__ key_mask, float scale, int H, int L, int P,
     half_t* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) float tab[64 * kGenStride];          // C2P [query][position]
-  __shared__ __attribute__((aligned(16))) half_t rows[kGenPass * 64];          // a pass's table rows (fused: V rows)
-  // Workgroup -> (b, h, query block qb, key block ky; the fused kernel takes
-  // every key block).  Workgroups go to the 8 XCDs round-robin; with H a
-  // multiple of 8, XCD x takes heads x H / 8 .. (x + 1) H / 8 - 1 only, so
-  // its L2 holds just those heads' index tensors and position tables.
-  constexpr int MAXKB = kGenKeyBlocks;
-  const int nqb = (L + 63) / 64, nky = (L / 16 + MAXKB - 1) / MAXKB;
-  const int nky_wg = FUSED ? 1 : nky;
-  int h, qb, ky, b;
+  constexpr int KB = kGenKeyBlocks;
+  __shared__ __attribute__((aligned(1024))) half_t rk[kGenWin * 64];    // window of posK rows
+  __shared__ __attribute__((aligned(1024))) half_t rq[kGenWin * 64];    // window of posQ rows
+  __shared__ __attribute__((aligned(1024))) half_t krows[64 * 64];      // K rows of the key block
+  __shared__ __attribute__((aligned(1024))) half_t vrows[2][64 * 64];   // V rows of this and the next key block
+  __shared__ __attribute__((aligned(16))) float tab[64 * kBiasStride];  // C2P [query][col], then P2C [key][col]
+  __shared__ int ranges[2][4][2 + 2 * KB];  // per wave: least c2p, -c2p, then p2c and -p2c of each 16-key block
+  // Workgroup -> (b, h, query block qb), heads to XCDs as in the bias kernel.
+  const int nqb = (L + 63) / 64, nky = nqb;
+  int h, qb, b;
   {
     const int w = blockIdx.x;
     int r;
@@ -181,385 +532,355 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FUSED ? 4 :
       r = w / H;
     }
     qb = r % nqb;
-    r /= nqb;
-    ky = r % nky_wg;
-    b = r / nky_wg;
+    b = r / nqb;
   }
-  const int bh = b * H + h;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lc = lane & 15, g = lane >> 4;
-  const int qw = qb * 64 + 16 * wave;  // the wave's first query
-  const bool active = qw < L;          // uniform
-  const int qg = qw + lc;              // this lane's query in the score tile (keys 4 g .. 4 g + 3 of a block)
-  const half_t* qbase = q + (int64_t)bh * L * 64;
-  const half_t* kbase = k + (int64_t)bh * L * 64;
+  const int qw = qb * 64 + 16 * wave;            // the wave's first query
+  const int qg = qw + lc;                        // this lane's query in the score tile (keys 4 g .. 4 g + 3 of a block)
+  const int qr = qg < L ? qg : L - 1;
   const half_t* pkh = pos_key + (int64_t)h * P * 64;
   const half_t* pqh = pos_query + (int64_t)h * P * 64;
   const int32_t* c2ph = c2p_idx + (int64_t)h * L * L;
   const int32_t* p2ch = p2c_idx + (int64_t)h * L * L;
   const half_t* mrow = key_mask + (int64_t)b * L;
-  const int qr = qg < L ? qg : L - 1;
-  const half8_t qf0 = *reinterpret_cast<const half8_t*>(qbase + (qr * 64 + 8 * g));
-  const half8_t qf1 = *reinterpret_cast<const half8_t*>(qbase + (qr * 64 + 32 + 8 * g));
+  const int64_t bh = (int64_t)b * H + h;
+  const half_t* kbase = k + bh * L * 64;
+  const half_t* vbase = v + bh * L * 64;
   auto clampi = [&](int x) { return x < 0 ? 0 : (x >= P ? P - 1 : x); };
-  auto unpack = [](const uint32_t (&w)[2], int j) -> int { return (int)((w[j >> 1] >> (16 * (j & 1))) & 0xFFFFu); };
+  auto key_of = [&](int kyb, int kb) { return 64 * kyb + 16 * kb + 4 * g; };  // this lane's first key of block kb
+  const half8_t q0 = *reinterpret_cast<const half8_t*>(q + bh * L * 64 + (uint32_t)(qr * 64 + 8 * g));
+  const half8_t q1 = *reinterpret_cast<const half8_t*>(q + bh * L * 64 + (uint32_t)(qr * 64 + 32 + 8 * g));
 
-  // Steps of a key block: the passes over the posK rows that hold any c2p
-  // index of the key block (passes c_lo .. c_lo + nc - 1), then the passes
-  // over the posQ rows that hold any of its p2c indices (p_lo .. p_lo + npp
-  // - 1); pass p covers table rows [64 p, + 64) (rows past P repeat row
-  // P - 1).  A pass holding no index of the block adds nothing, so it is not
-  // run (relative-position indices of a 64 x 64 tile span at most 127 rows:
-  // 2 or 3 passes of each table instead of all of them).  The fused kernel's
-  // last step brings the key block's V rows.  A step's rows are read into
-  // registers during the step before.
-  __shared__ int pass_range[4][4];  // per wave: least / greatest c2p and p2c index
-  int c_lo = 0, nc = 0, p_lo = 0, npp = 0;
-  constexpr int kPieces = kGenPass * 8 / 256;  // 16-byte pieces per thread
-  half8_t pre[kPieces];
-  auto fetch_rows = [&](int step, int ky_) {
+  // This lane's indices of a key block: c2p of keys key_of + j at query qr,
+  // p2c of query qr at those keys (keys past L: the last ones).
+  int ci[KB][4], pi[KB][4];
+  auto load_indices = [&](int kyb) {
 #pragma unroll
-    for (int it = 0; it < kPieces; ++it) {
-      const int i = t + 256 * it;
-      const int row = i >> 3, ch = i & 7;
-      if (step < nc + npp) {
-        const int prow0 = (step < nc ? c_lo + step : p_lo + step - nc) * kGenPass + row;
-        const half_t* src = (step < nc ? pkh : pqh) + (prow0 < P ? prow0 : P - 1) * 64;
-        pre[it] = *reinterpret_cast<const half8_t*>(src + ch * 8);
+    for (int kb = 0; kb < KB; ++kb) {
+      const int key = key_of(kyb, kb);
+      if constexpr (VEC) {
+        const int kc = key < L ? key : L - 4;
+        const int4 x = *reinterpret_cast<const int4*>(c2ph + (uint32_t)(qr * L + kc));
+        ci[kb][0] = x.x, ci[kb][1] = x.y, ci[kb][2] = x.z, ci[kb][3] = x.w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pi[kb][j] = p2ch[(uint32_t)((kc + j) * L + qr)];
       } else {
-        // V rows of keys past L are zeros (their probabilities are 0 too)
-        const int key = 16 * MAXKB * ky_ + row;
-        pre[it] = (half8_t){0, 0, 0, 0, 0, 0, 0, 0};
-        if (key < L) pre[it] = *reinterpret_cast<const half8_t*>(v + (int64_t)bh * L * 64 + (key * 64 + ch * 8));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int kc = key + j < L ? key + j : L - 1;
+          ci[kb][j] = c2ph[(uint32_t)(qr * L + kc)];
+          pi[kb][j] = p2ch[(uint32_t)(kc * L + qr)];
+        }
       }
     }
   };
+  half4_t mk[KB];
+  auto load_mask = [&](int kyb) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const int key = key_of(kyb, kb);
+      if constexpr (VEC) {
+        mk[kb] = *reinterpret_cast<const half4_t*>(mrow + (uint32_t)(key < L ? key : L - 4));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mk[kb][j] = mrow[(uint32_t)(key + j < L ? key + j : L - 1)];
+      }
+    }
+  };
+  // The clamped indices packed, c2p | p2c << 16, and the wave's index ranges
+  // to LDS.
+  auto put_ranges = [&](int buf, uint32_t (&cp)[KB][4]) {
+    int c_mn = P, c_mx = 0, p_mn[KB], p_mx[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      p_mn[kb] = P, p_mx[kb] = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = clampi(ci[kb][j]), p = clampi(pi[kb][j]);
+        c_mn = min(c_mn, c), c_mx = max(c_mx, c);
+        p_mn[kb] = min(p_mn[kb], p), p_mx[kb] = max(p_mx[kb], p);
+        cp[kb][j] = (uint32_t)c | ((uint32_t)p << 16);
+      }
+    }
+    int r[2 + 2 * KB];
+    r[0] = gen_wave_min(c_mn), r[1] = gen_wave_min(-c_mx);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) r[2 + 2 * kb] = gen_wave_min(p_mn[kb]), r[3 + 2 * kb] = gen_wave_min(-p_mx[kb]);
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < 2 + 2 * KB; ++i) ranges[buf][wave][i] = r[i];
+    }
+  };
+  // The tile's ranges (after a barrier): first row and last row of each
+  // window, the first c2p row of this wave and p2c row of each key block, and
+  // whether one window of each table serves every wave with kBiasTiles tiles.
+  struct Range {
+    int c_lo, c_hi, p_lo, p_hi, c_wave, p_own, p_block[KB];
+    bool single;
+  };
+  auto get_ranges = [&](int buf) -> Range {
+    Range x;
+    x.c_lo = P, x.c_hi = 0, x.p_lo = P, x.p_hi = 0, x.single = true;
+    x.c_wave = __builtin_amdgcn_readfirstlane(ranges[buf][wave][0]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int lo = __builtin_amdgcn_readfirstlane(ranges[buf][w][0]);
+      const int hi = -__builtin_amdgcn_readfirstlane(ranges[buf][w][1]);
+      x.c_lo = min(x.c_lo, lo), x.c_hi = max(x.c_hi, hi);
+      x.single = x.single && hi - lo < kBiasCols;
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      int lo = P, hi = P;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) lo = min(lo, ranges[buf][w][2 + 2 * kb]), hi = min(hi, ranges[buf][w][3 + 2 * kb]);
+      lo = __builtin_amdgcn_readfirstlane(lo), hi = -__builtin_amdgcn_readfirstlane(hi);
+      x.p_block[kb] = lo;
+      x.p_lo = min(x.p_lo, lo), x.p_hi = max(x.p_hi, hi);
+      x.single = x.single && hi - lo < kBiasCols;
+    }
+    x.single = x.single && x.c_hi - x.c_lo < kGenWin && x.p_hi - x.p_lo < kGenWin;
+    // the tiles stay inside the window
+    x.c_wave = min(x.c_wave, x.c_lo + kGenWin - kBiasCols);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) x.p_block[kb] = min(x.p_block[kb], x.p_lo + kGenWin - kBiasCols);
+    x.p_own = x.p_block[0];
+#pragma unroll
+    for (int kb = 1; kb < KB; ++kb) x.p_own = wave == kb ? x.p_block[kb] : x.p_own;
+    return x;
+  };
+  // DMA of `ROWS` rows, row r from src(r): lane l of a 1 KiB block brings
+  // physical chunk l % 8 of row l / 8.
+  auto issue_rows = [&](auto rows_c, half_t* dst, auto&& src) {
+    constexpr int BLOCKS = decltype(rows_c)::value / 32;  // 1 KiB blocks per wave
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j) {
+      const int blk = wave * BLOCKS + j;
+      const int row = 8 * blk + (lane >> 3);
+      load_lds16(src(row) + (((lane & 7) ^ ((row >> 1) & 7)) << 3), dst + blk * 512);
+    }
+  };
+  auto issue_window = [&](const half_t* table, half_t* dst, int base) {  // rows past P repeat row P - 1
+    issue_rows(std::integral_constant<int, kGenWin>{}, dst,
+               [&](int row) { return table + (uint32_t)((base + row < P ? base + row : P - 1) * 64); });
+  };
+  auto issue_block = [&](int kyb) {  // K rows (past L: the last one) and V rows (past L: zeros)
+    issue_rows(std::integral_constant<int, 64>{}, krows, [&](int row) {
+      const int key = 64 * kyb + row;
+      return kbase + (uint32_t)((key < L ? key : L - 1) * 64);
+    });
+    issue_rows(std::integral_constant<int, 64>{}, vrows[kyb & 1], [&](int row) {
+      const int key = 64 * kyb + row;
+      return key < L ? vbase + (uint32_t)(key * 64) : g_zero_row;
+    });
+  };
+  // kBiasTiles tiles of 16 window rows from row `r0` on against the 16 rows
+  // whose fragments are f0, f1, into this wave's table rows.
+  float* const own = tab + (16 * wave + lc) * kBiasStride;
+  auto products = [&](const half_t* win, int r0, half8_t f0, half8_t f1) {
+#pragma unroll
+    for (int tp = 0; tp < kBiasTiles; ++tp) {
+      const half8_t a0 = *reinterpret_cast<const half8_t*>(win + gen_swz(r0 + 16 * tp + lc, g));
+      const half8_t a1 = *reinterpret_cast<const half8_t*>(win + gen_swz(r0 + 16 * tp + lc, 4 + g));
+      float4_t r = {0.f, 0.f, 0.f, 0.f};
+      r = mfma16x16x32(a0, f0, r);
+      r = mfma16x16x32(a1, f1, r);  // lane: row lc, columns 16 tp + 4 g + i
+      *reinterpret_cast<float4_t*>(own + 16 * tp + 4 * g) = r;
+    }
+  };
+  auto c_of = [](uint32_t cp) { return (int)(cp & 0xFFFFu); };
+  auto p_of = [](uint32_t cp) { return (int)(cp >> 16); };
 
-  // fused: running max (per query row, the same in the row's four lanes),
-  // this lane's part of the row sum, and O^T (lane: query lc, d 16 dt + 4 g + i)
+  // running max (per query row, the same in the row's four lanes), this
+  // lane's part of the row sum, and O^T (lane: query lc, d 16 dt + 4 g + i)
   float m_run = -65504.f, l_run = 0.f;
   float4_t o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = (float4_t){0.f, 0.f, 0.f, 0.f};
 
-  if (t < 64) tab[t * kGenStride + kGenPass] = -0.0f;  // visible after the first step's barriers
-  for (int kyi = 0; kyi < (FUSED ? nky : 1); ++kyi) {  // uniform
-    const int kyb = FUSED ? kyi : ky;
-    const int kb0 = MAXKB * kyb;  // first 16-key block of this key block
-    const int nkb = L / 16 - kb0 < MAXKB ? L / 16 - kb0 : MAXKB;
-    // This lane's indices, clamped and packed two per register: c2p of keys
-    // 16 kb + 4 g + j at query qg, p2c of query qg at those keys.
-    uint32_t c2pk[MAXKB][2], p2ck[MAXKB][2];
-    int cmn = P, cmx = -1, pmn = P, pmx = -1;  // this lane's index range (valid scores only)
-#pragma unroll
-    // L is a multiple of 16, so a wave's queries all exist or none does: `ok`
-    // is uniform.  Blocks past nkb and waves past L load the indices of block
-    // nkb - 1 / query lc, in bounds and never used.
-    for (int kb = 0; kb < MAXKB; ++kb) {
-      const bool ok = active && kb < nkb;
-      const int kbc = kb < nkb ? kb : nkb - 1, qc = active ? qg : lc;
-      int pi[4];
-      const int4 ci = *reinterpret_cast<const int4*>(c2ph + (qc * L + 16 * (kb0 + kbc) + 4 * g));
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pi[j] = p2ch[(16 * (kb0 + kbc) + 4 * g + j) * L + qc];
-      const int c[4] = {clampi(ci.x), clampi(ci.y), clampi(ci.z), clampi(ci.w)};
-      const int pc[4] = {clampi(pi[0]), clampi(pi[1]), clampi(pi[2]), clampi(pi[3])};
-      c2pk[kb][0] = (uint32_t)c[0] | ((uint32_t)c[1] << 16);
-      c2pk[kb][1] = (uint32_t)c[2] | ((uint32_t)c[3] << 16);
-      p2ck[kb][0] = (uint32_t)pc[0] | ((uint32_t)pc[1] << 16);
-      p2ck[kb][1] = (uint32_t)pc[2] | ((uint32_t)pc[3] << 16);
-      if (ok) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          cmn = min(cmn, c[j]), cmx = max(cmx, c[j]);
-          pmn = min(pmn, pc[j]), pmx = max(pmx, pc[j]);
-        }
-      }
+  uint32_t cp[KB][4], cpn[KB][4];  // this block's and the next one's indices
+  load_indices(0);
+  issue_block(0);
+  load_mask(0);
+  put_ranges(0, cp);
+  stage_barrier();
+  Range rg = get_ranges(0);
+  if (rg.single) {
+    issue_window(pkh, rk, rg.c_lo);
+    issue_window(pqh, rq, rg.p_lo);
+  }
+  if (nky > 1) load_indices(1);
+  for (int kyi = 0; kyi < nky; ++kyi) {  // uniform
+    wait_vmcnt<0>();  // this block's windows, K and V rows
+    stage_barrier();  // (and every wave is done with the last block's P2C rows)
+    const bool more = kyi + 1 < nky;  // uniform
+    if (more) {
+      put_ranges((kyi + 1) & 1, cpn);
+      if (kyi + 2 < nky) load_indices(kyi + 2);
     }
-    // The workgroup's index range: wave reductions, then the four waves'
-    // through LDS (the previous key block read pass_range before its steps).
+    float acc[KB][4];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      cmn = min(cmn, __shfl_xor(cmn, off, 64)), cmx = max(cmx, __shfl_xor(cmx, off, 64));
-      pmn = min(pmn, __shfl_xor(pmn, off, 64)), pmx = max(pmx, __shfl_xor(pmx, off, 64));
+    for (int kb = 0; kb < KB; ++kb) {
+      float4_t r = {0.f, 0.f, 0.f, 0.f};
+      r = mfma16x16x32(*reinterpret_cast<const half8_t*>(krows + gen_swz(16 * kb + lc, g)), q0, r);
+      r = mfma16x16x32(*reinterpret_cast<const half8_t*>(krows + gen_swz(16 * kb + lc, 4 + g)), q1, r);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[kb][j] = r[j];  // lane: query lc, keys 16 kb + 4 g + j
     }
-    if (lane == 0) {
-      pass_range[wave][0] = cmn, pass_range[wave][1] = cmx;
-      pass_range[wave][2] = pmn, pass_range[wave][3] = pmx;
-    }
-    __syncthreads();
+    const half8_t kp0 = *reinterpret_cast<const half8_t*>(krows + gen_swz(16 * wave + lc, g));
+    const half8_t kp1 = *reinterpret_cast<const half8_t*>(krows + gen_swz(16 * wave + lc, 4 + g));
+    half4_t mkb[KB];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      cmn = min(cmn, pass_range[w][0]), cmx = max(cmx, pass_range[w][1]);
-      pmn = min(pmn, pass_range[w][2]), pmx = max(pmx, pass_range[w][3]);
-    }
-    // (wave 0's queries exist and nkb >= 1, so both ranges are non-empty)
-    c_lo = __builtin_amdgcn_readfirstlane(cmn / kGenPass);
-    nc = __builtin_amdgcn_readfirstlane(cmx / kGenPass) - c_lo + 1;
-    p_lo = __builtin_amdgcn_readfirstlane(pmn / kGenPass);
-    npp = __builtin_amdgcn_readfirstlane(pmx / kGenPass) - p_lo + 1;
-    const int nsteps = nc + npp + (FUSED ? 1 : 0);
-    fetch_rows(0, kyb);  // lands during the K loads and q.k
-    // K of the key block (keys past L clamped to L - 1).  Each wave keeps
-    // the fragments of its p2c keys (16 kb + lc, kb = 4 kg + wave) in
-    // registers: the bias kernel loads them from global memory; the fused
-    // kernel, whose q.k needs every key in every wave, stages the key block's
-    // K rows in the table-rows buffer first (the previous key block's last
-    // reads of that buffer, its V rows, came before this block's pass_range
-    // barrier; the first step's barrier follows these reads).
-    half8_t kp[MAXKB / 4][2];
-    float acc[MAXKB][4];
-    if constexpr (FUSED) {
+    for (int kb = 0; kb < KB; ++kb) mkb[kb] = mk[kb];
+    if (rg.single) {
+      products(rk, rg.c_wave - rg.c_lo, q0, q1);
+      wave_lds_sync();
 #pragma unroll
-      for (int it = 0; it < 16 * MAXKB * 8 / 256; ++it) {
-        const int i = t + 256 * it;
-        const int row = i >> 3, ch = i & 7;
-        const int key = 16 * kb0 + row < L ? 16 * kb0 + row : L - 1;
-        *reinterpret_cast<half8_t*>(rows + gen_swz(row, ch)) =
-            *reinterpret_cast<const half8_t*>(kbase + (key * 64 + ch * 8));
-      }
-      __syncthreads();  // K rows visible
-      // q.k of this wave's queries (lane: query lc, keys 16 kb + 4 g + i)
+      for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int kb = 0; kb < MAXKB; ++kb) {
-        const half8_t kf0 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * kb + lc, g));
-        const half8_t kf1 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * kb + lc, 4 + g));
-        float4_t r = {0.f, 0.f, 0.f, 0.f};
-        r = mfma16x16x32(kf0, qf0, r);
-        r = mfma16x16x32(kf1, qf1, r);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[kb][j] = r[j];
-      }
-#pragma unroll
-      for (int kg = 0; kg < MAXKB / 4; ++kg) {
-        kp[kg][0] = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * (4 * kg + wave) + lc, g));
-        kp[kg][1] = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * (4 * kg + wave) + lc, 4 + g));
-      }
+        for (int j = 0; j < 4; ++j) acc[kb][j] += own[c_of(cp[kb][j]) - rg.c_wave];
+      wave_lds_sync();
+      products(rq, rg.p_own - rg.p_lo, kp0, kp1);
     } else {
+      // Tiles wider than one window or one wave's columns: 80 columns of
+      // each table in turn, a position outside them reading a -0 column
+      // (x + -0 = x for every fp32 x).
+      if (lane < 16) own[kBiasCols] = -0.0f;
+      for (int w0 = rg.c_lo; w0 <= rg.c_hi; w0 += kBiasCols) {  // uniform
+        issue_window(pkh, rk, w0);
+        wait_vmcnt<0>();
+        stage_barrier();
+        products(rk, 0, q0, q1);
+        wave_lds_sync();
 #pragma unroll
-      for (int kg = 0; kg < MAXKB / 4; ++kg) {
-        const int key = 16 * (kb0 + 4 * kg + wave) + lc < L ? 16 * (kb0 + 4 * kg + wave) + lc : L - 1;
-        kp[kg][0] = *reinterpret_cast<const half8_t*>(kbase + (key * 64 + 8 * g));
-        kp[kg][1] = *reinterpret_cast<const half8_t*>(kbase + (key * 64 + 32 + 8 * g));
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[kb][j] += own[min((uint32_t)(c_of(cp[kb][j]) - w0), (uint32_t)kBiasCols)];
+        stage_barrier();
       }
+      for (int w0 = rg.p_lo; w0 <= rg.p_hi; w0 += kBiasCols) {  // uniform
+        issue_window(pqh, rq, w0);
+        wait_vmcnt<0>();
+        stage_barrier();
+        products(rq, 0, kp0, kp1);
+        stage_barrier();
 #pragma unroll
-      for (int kb = 0; kb < MAXKB; ++kb)
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[kb][j] = -0.0f;
-    }
-
-    float* const p2c64 = tab;  // p2c steps: P2C of 64 keys [key][kGenStride] in the C2P table's space
-    for (int step = 0; step < nc + npp; ++step) {  // uniform
-      __syncthreads();  // the previous step is done with `rows` and the tables
-#pragma unroll
-      for (int it = 0; it < kPieces; ++it) {
-        const int i = t + 256 * it;
-        *reinterpret_cast<half8_t*>(rows + gen_swz(i >> 3, i & 7)) = pre[it];
-      }
-      __syncthreads();
-      if (step + 1 < nsteps) fetch_rows(step + 1, kyb);  // lands during this step
-      // The packed indices stay packed across steps: unpacking them once,
-      // outside the loop, would take 32 more registers.
-#pragma unroll
-      for (int kb = 0; kb < MAXKB; ++kb) {
-        asm volatile("" : "+v"(c2pk[kb][0]), "+v"(c2pk[kb][1]), "+v"(p2ck[kb][0]), "+v"(p2ck[kb][1]));
-      }
-      const int base = (step < nc ? c_lo + step : p_lo + step - nc) * kGenPass;
-      if (step < nc) {
-        // ---- c2p: C2P of this wave's queries, gathered by the wave itself ----
-        if (active) {
-#pragma unroll
-          for (int tp = 0; tp < kGenPass / 16; ++tp) {
-            const half8_t a0 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * tp + lc, g));
-            const half8_t a1 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * tp + lc, 4 + g));
-            float4_t r = {0.f, 0.f, 0.f, 0.f};
-            r = mfma16x16x32(a0, qf0, r);
-            r = mfma16x16x32(a1, qf1, r);  // lane: query lc, positions 16 tp + 4 g + i
-            *reinterpret_cast<float4_t*>(tab + (16 * wave + lc) * kGenStride + 16 * tp + 4 * g) = r;
-          }
-          wave_lds_sync();
-          // Every score gathers a term; one whose position lies outside this
-          // pass reads the row's -0 column, which leaves the sum unchanged.
-          // (Blocks past nkb gather too, at index 0: their scores are never used.)
-          const float* const trow = tab + (16 * wave + lc) * kGenStride;
-#pragma unroll
-          for (int kb = 0; kb < MAXKB; ++kb)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[kb][j] += trow[gen_col(unpack(c2pk[kb], j) - base)];
-        }
-      } else {
-        // ---- p2c: P2C of 64 keys at a time (wave w: key block 4 kg + w) ----
-#pragma unroll
-        for (int kg = 0; kg < MAXKB / 4; ++kg) {
-          if (4 * kg >= nkb) continue;  // uniform
-          {
-            // (blocks past nkb hold clamped keys; their P2C rows are never read)
-            const half8_t kf0 = kp[kg][0], kf1 = kp[kg][1];
-#pragma unroll
-            for (int tp = 0; tp < kGenPass / 16; ++tp) {
-              const half8_t a0 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * tp + lc, g));
-              const half8_t a1 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * tp + lc, 4 + g));
-              float4_t r = {0.f, 0.f, 0.f, 0.f};
-              r = mfma16x16x32(a0, kf0, r);
-              r = mfma16x16x32(a1, kf1, r);  // lane: key lc, positions 16 tp + 4 g + i
-              *reinterpret_cast<float4_t*>(p2c64 + (16 * wave + lc) * kGenStride + 16 * tp + 4 * g) = r;
-            }
-          }
-          __syncthreads();
-          if (active) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                acc[4 * kg + u][j] += p2c64[(16 * u + 4 * g + j) * kGenStride + gen_col(unpack(p2ck[4 * kg + u], j) - base)];
-          }
-          __syncthreads();
-        }
+          for (int j = 0; j < 4; ++j)
+            acc[kb][j] +=
+                tab[(16 * kb + 4 * g + j) * kBiasStride + min((uint32_t)(p_of(cp[kb][j]) - w0), (uint32_t)kBiasCols)];
+        stage_barrier();
       }
     }
+    stage_barrier();  // P2C rows visible; every wave is done with both windows and the K rows
+    const Range now = rg;
+    if (more) {
+      rg = get_ranges((kyi + 1) & 1);
+      if (rg.single) {
+        issue_window(pkh, rk, rg.c_lo);
+        issue_window(pqh, rq, rg.p_lo);
+      }
+      issue_block(kyi + 1);
+      load_mask(kyi + 1);
+    }
+    if (now.single) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[kb][j] += tab[(16 * kb + 4 * g + j) * kBiasStride + (p_of(cp[kb][j]) - now.p_block[kb])];
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cp[kb][j] = cpn[kb][j];
 
-    if constexpr (!FUSED) {
-      // ---- scores: (c2p + p2c) * scale, masked keys -65504 ----
-      if (active) {  // (uniform: every lane of the wave takes part in the row swaps)
-        half_t* orow = out + (int64_t)bh * L * L + qg * L;
-        // Lane (g, query lc) holds keys 4 g .. 4 g + 3 of each 16-key block.
-        // Per group of four blocks a 4 x 4 transpose across the wave's four
-        // 16-lane rows (v_permlane32_swap, then v_permlane16_swap) leaves row
-        // g with all 16 keys of block 4 m + g, stored as one 32-byte piece.
+    // ---- online softmax over this key block, then P . V ----
+    constexpr float kLog2e = 1.4426950408889634f;
+    float bmax = m_run;
 #pragma unroll
-        for (int m = 0; m < MAXKB / 4; ++m) {
-          if (4 * m >= nkb) continue;  // uniform
-          uint32_t x[4][2];
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int kb = 4 * m + u, kbc = kb < nkb ? kb : nkb - 1;  // blocks past nkb: in bounds, never stored
-            const half4_t mk = *reinterpret_cast<const half4_t*>(mrow + 16 * (kb0 + kbc) + 4 * g);
-            half4_t sv;
+      for (int j = 0; j < 4; ++j) {
+        float sc = (float)mkb[kb][j] < -60000.f ? -65504.f : acc[kb][j] * scale;
+        if (key_of(kyi, kb) + j >= L) sc = -__builtin_inff();
+        acc[kb][j] = sc;
+        bmax = fmaxf(bmax, sc);
+      }
+    bmax = rows_max(bmax);
+    // exp(s - m) = 2^(s log2e - m log2e); the rounding of m log2e scales a
+    // whole row alike and cancels in the normalisation.
+    const float alpha = __builtin_amdgcn_exp2f(m_run * kLog2e - bmax * kLog2e);
+    m_run = bmax;
+    const float m_l2 = bmax * kLog2e;
+    l_run *= alpha;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const float sc = acc[kb][j] * scale;
-              sv[j] = (float)mk[j] < -60000.f ? (half_t)-65504.f : (half_t)sc;
-            }
-            const uint2 w = __builtin_bit_cast(uint2, sv);
-            x[u][0] = w.x, x[u][1] = w.y;
+    for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(acc[kb][j], kLog2e, -m_l2));
+        acc[kb][j] = e;
+        l_run += e;
+      }
+    {
+      // ds_read_b64_tr_b16: in each 16-lane group, source lane s names 4
+      // consecutive halfs and lane j receives element j % 4 of source lanes
+      // j / 4, 4 + j / 4, 8 + j / 4, 12 + j / 4.  Source lane lc of group g
+      // names V[16 T + 4 g + lc / 4][16 dt + 4 (lc % 4) ..], so lane (g, lc)
+      // receives V[16 T + 4 g + i][16 dt + lc], i = 0..3 (from 16 rows on,
+      // tile T + 1): with V as the A operand and P^T as the B operand the
+      // product lane holds O[query lc][16 dt + 4 g + i].  The swizzle term
+      // (row >> 1) & 7 of those rows is (2 g + lc / 8) & 7.
+      gen_lds_half_t* const rows3 = (gen_lds_half_t*)(lds_void_t*)vrows[kyi & 1];
+      const int tr_sw = (2 * g + (lc >> 3)) & 7;
+      const int tr_lane = (4 * g + (lc >> 2)) * 64 + 4 * (lc & 1);
+      const int tr_c = (lc >> 1) & 1;
+#pragma unroll
+      for (int T = 0; T < KB; T += 2) {
+        half8_t pa, pl;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; i += 2) {
+            const float x0 = acc[T + u][i], x1 = acc[T + u][i + 1];
+            const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+            pa[4 * u + i] = hi[0];
+            pa[4 * u + i + 1] = hi[1];
+            pl[4 * u + i] = (half_t)(x0 - (float)hi[0]);
+            pl[4 * u + i + 1] = (half_t)(x1 - (float)hi[1]);
           }
 #pragma unroll
-          for (int d = 0; d < 2; ++d) {
-            const auto s02 = __builtin_amdgcn_permlane32_swap(x[0][d], x[2][d], false, false);
-            const auto s13 = __builtin_amdgcn_permlane32_swap(x[1][d], x[3][d], false, false);
-            const uint32_t z0 = s02[0], z2 = s02[1], z1 = s13[0], z3 = s13[1];
-            const auto s01 = __builtin_amdgcn_permlane16_swap(z0, z1, false, false);
-            const auto s23 = __builtin_amdgcn_permlane16_swap(z2, z3, false, false);
-            x[0][d] = s01[0], x[1][d] = s01[1], x[2][d] = s23[0], x[3][d] = s23[1];
+        for (int dt = 0; dt < 4; ++dt) {
+          const gen_lds_half_t* a = rows3 + 16 * T * 64 + tr_lane + (((2 * dt + tr_c) ^ tr_sw) << 3);
+          const gen_short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)a);
+          const gen_short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)(a + 16 * 64));
+          const half4_t h0 = __builtin_bit_cast(half4_t, v0), h1 = __builtin_bit_cast(half4_t, v1);
+          half8_t vb;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            vb[i] = h0[i];
+            vb[4 + i] = h1[i];
           }
-          if (4 * m + g < nkb) {
-            half_t* dst = orow + 16 * (kb0 + 4 * m + g);
-            *reinterpret_cast<uint4*>(dst) = uint4{x[0][0], x[0][1], x[1][0], x[1][1]};
-            *reinterpret_cast<uint4*>(dst + 8) = uint4{x[2][0], x[2][1], x[3][0], x[3][1]};
-          }
+          o[dt] = mfma16x16x32(vb, pa, o[dt]);
+          o[dt] = mfma16x16x32(vb, pl, o[dt]);
         }
       }
-    } else {
-      // ---- online softmax over this key block, then P . V ----
-      constexpr float kLog2e = 1.4426950408889634f;
-      float bmax = m_run;
-#pragma unroll
-      for (int kb = 0; kb < MAXKB; ++kb) {
-        if (kb >= nkb) continue;  // uniform
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int key = 16 * (kb0 + kb) + 4 * g + j;
-          const float sc = (float)mrow[key] < -60000.f ? -65504.f : acc[kb][j] * scale;
-          acc[kb][j] = sc;
-          bmax = fmaxf(bmax, sc);
-        }
-      }
-      bmax = rows_max(bmax);
-      // exp(s - m) = 2^(s log2e - m log2e); the rounding of m log2e scales a
-      // whole row alike and cancels in the normalisation.
-      const float alpha = __builtin_amdgcn_exp2f(m_run * kLog2e - bmax * kLog2e);
-      m_run = bmax;
-      const float m_l2 = bmax * kLog2e;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
-#pragma unroll
-      for (int kb = 0; kb < MAXKB; ++kb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float e = kb < nkb ? __builtin_amdgcn_exp2f(fmaf(acc[kb][j], kLog2e, -m_l2)) : 0.f;
-          acc[kb][j] = e;
-          l_run += e;
-        }
-      // V step: the key block's V rows into `rows` (every wave's p2c reads
-      // of `rows` ended at the last step's closing barrier)
-#pragma unroll
-      for (int it = 0; it < kPieces; ++it) {
-        const int i = t + 256 * it;
-        *reinterpret_cast<half8_t*>(rows + gen_swz(i >> 3, i & 7)) = pre[it];
-      }
-      __syncthreads();
-      if (active) {
-        // ds_read_b64_tr_b16: in each 16-lane group, source lane s names 4
-        // consecutive halfs and lane j receives element j % 4 of source lanes
-        // j / 4, 4 + j / 4, 8 + j / 4, 12 + j / 4.  Source lane lc of group g
-        // names V[16 T + 4 g + lc / 4][16 dt + 4 (lc % 4) ..], so lane (g, lc)
-        // receives V[16 T + 4 g + i][16 dt + lc], i = 0..3 (from 16 rows on,
-        // tile T + 1): with V as the A operand and P^T as the B operand the
-        // product lane holds O[query lc][16 dt + 4 g + i].  The swizzle term
-        // (row >> 1) & 7 of those rows is (2 g + lc / 8) & 7.
-        gen_lds_half_t* const rows3 = (gen_lds_half_t*)(gen_lds_void_t*)rows;
-        const int tr_sw = (2 * g + (lc >> 3)) & 7;
-        const int tr_lane = (4 * g + (lc >> 2)) * 64 + 4 * (lc & 1);
-        const int tr_c = (lc >> 1) & 1;
-#pragma unroll
-        for (int T = 0; T < MAXKB; T += 2) {
-          if (T >= nkb) continue;  // uniform; a tile T + 1 past nkb has P = 0 and zero V rows
-          half8_t pa, pl;
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-              const float x0 = acc[T + u][i], x1 = acc[T + u][i + 1];
-              const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-              pa[4 * u + i] = hi[0];
-              pa[4 * u + i + 1] = hi[1];
-              pl[4 * u + i] = (half_t)(x0 - (float)hi[0]);
-              pl[4 * u + i + 1] = (half_t)(x1 - (float)hi[1]);
-            }
-#pragma unroll
-          for (int dt = 0; dt < 4; ++dt) {
-            const gen_lds_half_t* a = rows3 + 16 * T * 64 + tr_lane + (((2 * dt + tr_c) ^ tr_sw) << 3);
-            const gen_short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)a);
-            const gen_short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)(a + 16 * 64));
-            const half4_t h0 = __builtin_bit_cast(half4_t, v0), h1 = __builtin_bit_cast(half4_t, v1);
-            half8_t vb;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              vb[i] = h0[i];
-              vb[4 + i] = h1[i];
-            }
-            o[dt] = mfma16x16x32(vb, pa, o[dt]);
-            o[dt] = mfma16x16x32(vb, pl, o[dt]);
-          }
-        }
-      }
-      // The next key block writes pass_range and `rows` only after barriers
-      // that every wave reaches after its V reads here.
     }
   }
-  if constexpr (FUSED) {
-    if (active && qg < L) {
-      const float inv = 1.0f / rows_sum(l_run);
-      half_t* orow = out + (((int64_t)b * L + qg) * H + h) * 64;
+  if (qg < L) {
+    const float inv = 1.0f / rows_sum(l_run);
+    half_t* orow = out + (((int64_t)b * L + qg) * H + h) * 64;
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        half4_t ov;
+    for (int dt = 0; dt < 4; ++dt) {
+      half4_t ov;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ov[i] = (half_t)(o[dt][i] * inv);
-        *reinterpret_cast<half4_t*>(orow + 16 * dt + 4 * g) = ov;
-      }
+      for (int i = 0; i < 4; ++i) ov[i] = (half_t)(o[dt][i] * inv);
+      *reinterpret_cast<half4_t*>(orow + 16 * dt + 4 * g) = ov;
     }
   }
 }
@@ -569,13 +890,13 @@ __global__ void relative_index_table_kernel(int32_t* __restrict__ out, int n, in
   if (i < 2 * n - 1) out[i] = relative_index(i - (n - 1), bucket_size, max_position);
 }
 
-// The matrix-core kernels read q, k, v and the table rows in 16-byte pieces,
-// the c2p indices and (the bias kernel) the key mask four at a time, and
-// store 8- or 16-byte pieces of the output; both entry points hold every
+// The matrix-core kernels read q, k, v and the table rows in 16-byte pieces
+// and, where L allows, the c2p indices and the key mask four at a time, and
+// store pieces of up to 16 bytes of the output; both entry points hold every
 // operand to 16-byte alignment, as the header states.
 bool general_mfma_ok(int64_t D, int64_t L, int64_t P, const int32_t* error_flag,
                      std::initializer_list<const void*> ptrs) {
-  if (D != 64 || L % 16 != 0 || L > 512 || P > 65536 || error_flag != nullptr) return false;
+  if (D != 64 || L > 512 || P > 65536 || error_flag != nullptr) return false;
   for (const void* p : ptrs)
     if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
   return true;
@@ -588,13 +909,27 @@ int launch_relative_bias_general(const void* q, const void* k, const void* pos_k
                                  int64_t H, int64_t L, int64_t D, int64_t P, void* out, int32_t* error_flag,
                                  hipStream_t stream) {
   if (B * H * L == 0) return GD_OK;
-  // Indices travel packed in 16 bits, so the tables hold at most 65536 rows.
   if (general_mfma_ok(D, L, P, error_flag, {q, k, pos_key, pos_query, c2p, p2c, key_mask, out})) {
-    const dim3 grid((unsigned)(B * H * ((L + 63) / 64) * ((L / 16 + kGenKeyBlocks - 1) / kGenKeyBlocks)));
-    hipLaunchKernelGGL(general_mfma_kernel<false>, grid, dim3(256), 0, stream, static_cast<const half_t*>(q),
-                       static_cast<const half_t*>(k), nullptr, static_cast<const half_t*>(pos_key),
+    // Batch rows per workgroup: the fewest that leave one round of the two
+    // workgroups a CU holds (a single one takes the form of three per CU).  A workgroup's indices and table rows cost it about
+    // 7 us and each batch row 2 us (B = 32, L = 256, 8,192 tiles: 1, 2, 4, 8, 16
+    // and 32 rows per workgroup take 133, 81, 55, 43, 36 and 45 us).
+    const int64_t blocks = (L + 63) / 64, tiles = H * blocks * blocks, slots = 2 * kGenCus;
+    const int64_t want = std::min(B, (B * tiles + slots - 1) / slots);
+    const int64_t nb = (B + (B + want - 1) / want - 1) / ((B + want - 1) / want);  // in even groups
+    const dim3 grid((unsigned)(tiles * ((B + nb - 1) / nb)));
+    auto pick = [&](auto multi) {
+      constexpr bool M = decltype(multi)::value;
+      return L % 8 == 0   ? relative_bias_mfma_kernel<8, M>
+             : L % 4 == 0 ? relative_bias_mfma_kernel<4, M>
+             : L % 2 == 0 ? relative_bias_mfma_kernel<2, M>
+                          : relative_bias_mfma_kernel<1, M>;
+    };
+    const auto kernel = nb > 1 ? pick(std::true_type{}) : pick(std::false_type{});
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const half_t*>(q),
+                       static_cast<const half_t*>(k), static_cast<const half_t*>(pos_key),
                        static_cast<const half_t*>(pos_query), c2p, p2c, static_cast<const half_t*>(key_mask), scale,
-                       (int)H, (int)L, (int)P, static_cast<half_t*>(out));
+                       (int)B, (int)H, (int)L, (int)P, (int)nb, static_cast<half_t*>(out));
     GD_LAUNCH_CHECK();
     return GD_OK;
   }
@@ -612,10 +947,10 @@ int launch_fused_attention_general(const void* q, const void* k, const void* v, 
                                    float scale, int64_t B, int64_t H, int64_t L, int64_t D, int64_t P, void* out,
                                    int32_t* error_flag, hipStream_t stream) {
   if (B * H * L == 0) return GD_OK;
-  // Indices travel packed in 16 bits, so the tables hold at most 65536 rows.
   if (general_mfma_ok(D, L, P, error_flag, {q, k, v, pos_key, pos_query, c2p, p2c, key_mask, out})) {
     const dim3 grid((unsigned)(B * H * ((L + 63) / 64)));
-    hipLaunchKernelGGL(general_mfma_kernel<true>, grid, dim3(256), 0, stream, static_cast<const half_t*>(q),
+    const auto kernel = L % 4 == 0 ? fused_attention_mfma_kernel<true> : fused_attention_mfma_kernel<false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const half_t*>(q),
                        static_cast<const half_t*>(k), static_cast<const half_t*>(v),
                        static_cast<const half_t*>(pos_key), static_cast<const half_t*>(pos_query), c2p, p2c,
                        static_cast<const half_t*>(key_mask), scale, (int)H, (int)L, (int)P,

@@ -173,6 +173,15 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// One 1 KiB block straight from global memory into LDS: lane l of the wave
+// brings 16 bytes from its own address g to lds_block + 16 l (lds_block is the
+// same in every lane).
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+__device__ __forceinline__ void load_lds16(const half_t* g, half_t* lds_block) {
+  __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(g), (lds_void_t*)(lds_block), 16, 0, 0);
+}
+
 // MFMA wrappers (gfx950 double-rate fp16 forms).
 //  16x16x32: A lane l -> row l%16, k = 8*(l/16)+[0,8); B lane l -> col l%16,
 //            same k; C lane l -> col l%16, rows 4*(l/16)+[0,4).

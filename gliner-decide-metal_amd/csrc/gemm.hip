@@ -268,12 +268,6 @@ __global__ __launch_bounds__(kThreads) void gemm_nt_kernel(const half_t* __restr
 // 8-byte store per group and writes coalesced 8-byte row pieces.
 // ---------------------------------------------------------------------------
 
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-__device__ __forceinline__ void load_lds16(const half_t* g, half_t* lds_block) {
-  __builtin_amdgcn_global_load_lds(reinterpret_cast<const void*>(g), (lds_void_t*)(lds_block), 16, 0, 0);
-}
-
 
 // LDS layout of one operand tile: rows of BK halfs; the 16-byte chunk index
 // is XORed with the row's position inside its 256-byte bank line group, so a

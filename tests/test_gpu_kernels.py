@@ -672,6 +672,47 @@ def test_general_index_kernels_random_indices(L, P, H):
                                atol=2e-3)
 
 
+@pytest.mark.parametrize("L,P,H,B,relative", [
+    (1, 512, 2, 2, True), (3, 40, 1, 2, False), (17, 512, 8, 3, True), (50, 512, 2, 9, True), (63, 300, 3, 2, False),
+    (65, 512, 2, 3, True), (130, 200, 2, 2, False), (200, 512, 8, 3, True), (201, 512, 2, 2, True),
+    (333, 512, 1, 2, False), (511, 512, 1, 1, True), (317, 512, 16, 7, True)])
+def test_general_index_kernels_any_length(L, P, H, B, relative):
+    """The matrix-core general-index kernels at lengths that are no multiple
+    of a tile, of 8, of 4 or of 2 (partial key and query blocks, unaligned
+    output rows, waves with no query), with relative-position indices (one
+    table window per tile) and arbitrary ones (several windows); at L = 317 the
+    bias kernel walks the 7 batch rows in groups of 4 and 3.  The last
+    batch row has every key masked."""
+    r = np.random.default_rng(1700 + L)
+    q, k, v = (r.standard_normal((B, H, L, 64)).astype(np.float16) for _ in range(3))
+    pkh, pqh = (r.standard_normal((H, P, 64)).astype(np.float16) for _ in range(2))
+    if relative:
+        rel = np.arange(L)[:, None] - np.arange(L)[None, :]
+        idx = np.clip(O.relative_bucket(rel) + 256, 0, P - 1).astype(np.int32)
+        c2p = np.ascontiguousarray(np.broadcast_to(idx, (H, L, L)))
+        p2c = np.ascontiguousarray(np.broadcast_to(idx.T, (H, L, L)))
+    else:
+        c2p = r.integers(0, P, size=(H, L, L)).astype(np.int32)
+        p2c = r.integers(0, P, size=(H, L, L)).astype(np.int32)
+    lengths = np.array([L] + [max(1, L // 3)] * (B - 2) + [0])[:B]
+    key_mask = np.where(np.arange(L)[None, :] < lengths[:, None], 0.0, -65504.0).astype(np.float16)
+    scale = O.scale_f32(64)
+    args = [dev(a) for a in (q, k, v, pkh, pqh, c2p, p2c, key_mask)]
+    want = O.relative_bias_kernel(q, k, pkh, pqh, c2p, p2c, key_mask, scale)
+    got = host(fk().relative_bias(*args[:2], *args[3:], scale, B, H, L, 64, P))
+    masked = np.broadcast_to(key_mask[:, None, None, :] < -60000, got.shape)
+    assert np.all(got[masked] == -65504.0)
+    # an fp32 sum of 129 products (8 units of 2^-24 per MFMA step of the terms' magnitudes, as above), one rounding
+    acc = 4.0 * 8.0 * 2.0 ** -24 * O.relative_bias_kernel(np.abs(q), np.abs(k), np.abs(pkh), np.abs(pqh), c2p, p2c,
+                                                            np.zeros_like(key_mask), scale, round16=False)
+    err = np.abs(got - want)[~masked]
+    bound = (np.maximum(ulp16(got), ulp16(want)) + acc)[~masked]
+    assert np.all(err <= bound + 1e-12), (err - bound).max()
+    want = O.fused_attention_kernel(q, k, v, pkh, pqh, c2p, p2c, key_mask, scale)
+    got = host(fk().fused_attention(*args, scale, B, H, L, 64, P))
+    assert np.max(np.abs(got - want)) <= 2e-3  # one fp16 rounding of values below 4
+
+
 def test_general_index_kernels_clamp_out_of_range_indices():
     """Indices outside [0, P) read the nearest table row (the per-query
     kernels' rule, kept by the matrix-core kernels)."""
