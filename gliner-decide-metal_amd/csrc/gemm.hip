@@ -18,11 +18,13 @@
 //     through LDS into coalesced row segments; gemm_lds_split160_kernel is
 //     its 160 x 128 tile on eight waves of unequal row counts (bias
 //     epilogues);
-//   * gemm_skinny_kernel for at most 32 rows (one short sequence): 32 x 16
-//     tiles of two waves on v_mfma_f32_16x16x16_f16, eight 128-deep stages;
+//   * gemm_skinny_kernel for few rows (one text, the marker rows, a long sum
+//     on a few hundred): tiles of 32 x 16 to 64 x 32, a wave for each 16 x 16
+//     on v_mfma_f32_16x16x16_f16, four or eight 128-deep stages;
 //   * gemm_nt_kernel, register-staged (global -> registers -> LDS, one K step
-//     ahead): operands whose rows are gathered through an index list (the
-//     classifier's marker rows) or that exceed 32-bit element offsets.
+//     ahead): operands that exceed 32-bit element offsets.
+// Rows may be gathered through an index list (the classifier's marker rows):
+// the DMA kernels look each row up once, where they form its address.
 // Every kernel accumulates an element over the same 16-wide K slices in the
 // same order, so a row's bits do not depend on M or on the kernel chosen.
 // launch_linear chooses the kernel and tile: up to 4,096 rows by a cost model
@@ -125,7 +127,7 @@ __device__ __forceinline__ half_t epilogue(float acc, float b) {
 // BM x BN tile and walks K in steps of 64, global -> registers -> LDS double
 // buffered (the loads of step k + 1 in flight while the MFMAs of step k
 // run), each wave on a (BM/2) x (BN/2) sub-tile.  With GATHER, A row i is
-// row a_rows[i] of the operand (the classifier's marker rows).
+// row a_rows[i] of the operand.
 template <int BM, int BN, int EPI, bool GATHER>
 __global__ __launch_bounds__(kThreads) void gemm_nt_kernel(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                            const half_t* __restrict__ bias, half_t* __restrict__ C,
@@ -292,12 +294,26 @@ struct StageLayout {
 template <int V>
 using ic = std::integral_constant<int, V>;
 
-template <int BM, int BN, int WAVES_M, int BK, int NSTAGE, int EPI, int NW>
+// Operand row of output row m (rows past M repeat the last one): m itself, or
+// where the rows are gathered, rows[m] held to the operand's rows.
+struct PlainRows {
+  __device__ __forceinline__ int operator()(int m, int M) const { return m < M ? m : M - 1; }
+};
+struct GatheredRows {
+  const int32_t* rows;
+  int count;
+  __device__ __forceinline__ int operator()(int m, int M) const {
+    const int r = rows[m < M ? m : M - 1];
+    return r < 0 ? 0 : (r >= count ? count - 1 : r);
+  }
+};
+
+template <int BM, int BN, int WAVES_M, int BK, int NSTAGE, int EPI, int NW, class Rows>
 __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __restrict__ A,
                                                                 const half_t* __restrict__ W,
                                                                 const half_t* __restrict__ bias,
                                                                 half_t* __restrict__ C, int M, int N, int K,
-                                                                int64_t lda, int64_t ldc, int tiles_m, int tiles_n) {
+                                                                int64_t lda, int64_t ldc, int tiles_m, int tiles_n, Rows row_map) {
   using Lay = StageLayout<BK>;
   constexpr int NT = 64 * NW;  // threads
   constexpr int WAVES_N = NW / WAVES_M;
@@ -379,8 +395,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __re
 #pragma unroll
   for (int j = 0; j < A_BLK; ++j) {
     const int blk = wave * A_BLK + j;
-    int m = tile_m * BM + blk * Lay::kRowsPerBlock + lane / Lay::kChunks;
-    m = m < M ? m : M - 1;
+    const int m = row_map(tile_m * BM + blk * Lay::kRowsPerBlock + lane / Lay::kChunks, M);
     a_off[j] = (uint32_t)((int64_t)m * lda + Lay::dma_chunk(lane, blk) * 8);
   }
 #pragma unroll
@@ -663,15 +678,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __re
   store_rows(0, BM, [&](int r) { return rows_of(r / RPA) + (r % RPA) * BN; });
 }
 
-template <int BM, int BN, int WAVES_M, int BK, int NSTAGE, int NW = 8>
+template <int BM, int BN, int WAVES_M, int BK, int NSTAGE, int NW = 8, class Rows = PlainRows>
 int launch_lds_tile(const half_t* A, const half_t* W, const half_t* bias, half_t* C, int M, int N, int K, int64_t lda,
-                    int64_t ldc, int epi, hipStream_t stream) {
+                    int64_t ldc, int epi, hipStream_t stream, Rows rows = {}) {
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = N / BN;
   const dim3 grid(tiles_m * tiles_n), block(64 * NW);
 #define GD_LDS_GEMM(E)                                                                                               \
-  hipLaunchKernelGGL((gemm_nt_lds_kernel<BM, BN, WAVES_M, BK, NSTAGE, E, NW>), grid, block, 0, stream, A, W, bias, C, M, N, \
-                     K, lda, ldc, tiles_m, tiles_n)
+  hipLaunchKernelGGL((gemm_nt_lds_kernel<BM, BN, WAVES_M, BK, NSTAGE, E, NW, Rows>), grid, block, 0, stream, A, W, bias, C, M, N, \
+                     K, lda, ldc, tiles_m, tiles_n, rows)
   switch (epi) {
     case GD_EPI_NONE: GD_LDS_GEMM(GD_EPI_NONE); break;
     case GD_EPI_BIAS: GD_LDS_GEMM(GD_EPI_BIAS); break;
@@ -888,15 +903,16 @@ int launch_lds_tile_gelu320(const half_t* A, const half_t* W, const half_t* bias
                             int64_t lda, int64_t ldc, hipStream_t stream) {
   const int tiles_m = (M + 319) / 320;
   const int tiles_n = N / 256;
-  hipLaunchKernelGGL((gemm_nt_lds_kernel<320, 256, 2, 64, 2, GD_EPI_BIAS_GELU, 8>), dim3(tiles_m * tiles_n), dim3(512),
-                     0, stream, A, W, bias, C, M, N, K, lda, ldc, tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_nt_lds_kernel<320, 256, 2, 64, 2, GD_EPI_BIAS_GELU, 8, PlainRows>), dim3(tiles_m * tiles_n), dim3(512),
+                     0, stream, A, W, bias, C, M, N, K, lda, ldc, tiles_m, tiles_n, PlainRows{});
   GD_LAUNCH_CHECK();
   return GD_OK;
 }
 
-template <int BM, int BN, bool GATHER>
+template <bool GATHER>
 int launch_tile(const half_t* A, const half_t* W, const half_t* bias, half_t* C, int M, int N, int K, int64_t lda,
                 int64_t ldc, const int32_t* a_rows, int a_row_count, int epi, hipStream_t stream) {
+  constexpr int BM = 128, BN = 128;
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = N / BN;
   const dim3 grid(tiles_m * tiles_n), block(kThreads);
@@ -923,47 +939,51 @@ int launch_tile(const half_t* A, const half_t* W, const half_t* bias, half_t* C,
 }
 
 // ---------------------------------------------------------------------------
-// Skinny products: at most 32 rows (one short sequence, a few marker rows).
-// The time of such a product is the chain of dependent MFMAs per accumulator
-// (K / 16 of them) plus how fast the workgroups stream W; the tile kernels
-// above give N / 64 workgroups with one 32 x 32 accumulator per wave.  Here
-// a workgroup of two waves owns a 32 x 16 tile (N / 16 workgroups), wave w
-// rows 16 w .. 16 w + 15 in one v_mfma_f32_16x16x16_f16 chain, and keeps
-// eight 128-deep stages of A and W in flight (96 KiB).  The 16 x 16 x 16 MFMA
+// Skinny products: few rows (one text, marker rows, a long sum on a few
+// hundred).  The time of such a product is the chain of dependent MFMAs per
+// accumulator (K / 16 of them, 40 cycles each) plus how fast the workgroups
+// stream W; the tile kernels above give (M / 64) (N / 64) workgroups with one
+// 32 x 32 accumulator per wave.  Here a wave owns 16 x 16 in one
+// v_mfma_f32_16x16x16_f16 chain and a workgroup MB x NB of them, small enough
+// that the product is spread over the chip, with NST 128-deep stages of A and W
+// in flight (64 to 96 KiB).  FFN-down (K = 4096) at 64, 256 and 300 rows takes
+// 7.8, 8.1 and 10.2 us where the 64 x 64 tiles take 15.4 to 15.7; above a chain's
+// 4.3 us it is bound by what a CU draws from its L2.  The 16 x 16 x 16 MFMA
 // sums the same 16 products per K slice as the 32 x 32 x 16 form, bit for bit
 // (gd_diag_mfma_forms runs both on the device; a GPU test compares them over
 // wide-range, cancelling and large-accumulator operands), and the
 // slices run in the same order, so each element has the bits the tile
 // kernels give it.
 //
-// Stage layout: rows of 128 halfs (256 B), A rows 0..31 then W rows 32..47;
+// Stage layout: rows of 128 halfs (256 B), the tile's A rows, then its W rows;
 // the 16-byte chunk index is XORed with the row's low four bits, so the 16
 // rows of a fragment read at one logical chunk cover the 64 banks once.
 // ---------------------------------------------------------------------------
 constexpr int kSkBK = 128;                        // K per stage
-constexpr int kSkStages = 8;
-constexpr int kSkRows = 48;                       // 32 A rows + 16 W rows
-constexpr int kSkStage = kSkRows * kSkBK;         // halfs per stage
-constexpr int kSkLoads = kSkStage * 2 / 1024 / 2;  // 1 KiB DMA blocks per wave per stage (6)
-static_assert((kSkStages - 1) * kSkLoads < 64, "vmcnt range");
 
 __device__ __forceinline__ int sk_offset(int row, int chunk) { return row * kSkBK + ((chunk ^ (row & 15)) << 3); }
 
-template <int EPI>
-__global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restrict__ A, const half_t* __restrict__ W,
+// MB, NB: 16-row and 16-column blocks of the tile, a wave for each pair; NST:
+// stages in flight.
+template <int MB, int NB, int NST, int EPI, class Rows>
+__global__ __launch_bounds__(64 * MB * NB) void gemm_skinny_kernel(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                          const half_t* __restrict__ bias, half_t* __restrict__ C,
-                                                         int M, int N, int K, int64_t lda, int64_t ldc) {
+                                                         int M, int N, int K, int64_t lda, int64_t ldc,
+                                                         int tiles_m, Rows row_map) {
+  constexpr int kSkStage = 16 * (MB + NB) * kSkBK;              // halfs per stage: the A rows, then the W rows
+  constexpr int kSkLoads = kSkStage * 2 / 1024 / (MB * NB);        // 1 KiB DMA blocks per wave per stage
+  static_assert((NST - 1) * kSkLoads < 64 && kSkLoads * MB * NB * 512 == kSkStage, "vmcnt range, whole blocks");
+  static_assert(NST == 4 || NST == 8, "one named buffer per stage, two fragment sets");
   // One named array per stage: every LDS read names its buffer at compile
   // time, so the compiler's waits cover only the DMA into that buffer.
   __shared__ __attribute__((aligned(1024))) half_t sk0[kSkStage];
   __shared__ __attribute__((aligned(1024))) half_t sk1[kSkStage];
   __shared__ __attribute__((aligned(1024))) half_t sk2[kSkStage];
   __shared__ __attribute__((aligned(1024))) half_t sk3[kSkStage];
-  __shared__ __attribute__((aligned(1024))) half_t sk4[kSkStage];
-  __shared__ __attribute__((aligned(1024))) half_t sk5[kSkStage];
-  __shared__ __attribute__((aligned(1024))) half_t sk6[kSkStage];
-  __shared__ __attribute__((aligned(1024))) half_t sk7[kSkStage];
-  static_assert(kSkStages == 8, "one named buffer per stage");
+  __shared__ __attribute__((aligned(1024))) half_t sk4[NST > 4 ? kSkStage : 8];
+  __shared__ __attribute__((aligned(1024))) half_t sk5[NST > 4 ? kSkStage : 8];
+  __shared__ __attribute__((aligned(1024))) half_t sk6[NST > 4 ? kSkStage : 8];
+  __shared__ __attribute__((aligned(1024))) half_t sk7[NST > 4 ? kSkStage : 8];
   auto stage = [&](auto b) -> half_t* {
     constexpr int B = decltype(b)::value;
     if constexpr (B == 0) return sk0;
@@ -976,9 +996,14 @@ __global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restri
     else return sk7;
   };
 
-  const int tile_n = blockIdx.x;
+  // Workgroups go to the 8 XCDs round-robin: XCD x takes the x-th run of tiles,
+  // tile rows first, so its L2 reads its own columns of W once and no others.
+  const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, extra = gridDim.x & 7;
+  const int tile = xcd * per_xcd + (xcd < extra ? xcd : extra) + (blockIdx.x >> 3);
+  const int tile_m = tile % tiles_m, tile_n = tile / tiles_m;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave % MB, wn = wave / MB;  // 16 rows, 16 columns
   const int g = lane >> 4, r = lane & 15;
 
   // This lane's 16-byte pieces: block j of the wave (stage block 6 w + j)
@@ -992,12 +1017,11 @@ __global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restri
     const int blk = wave * kSkLoads + j;
     const int row = 4 * blk + (lane >> 4);
     const int chunk = (lane & 15) ^ (row & 15);
-    is_w[j] = row >= 32;
-    if (row < 32) {
-      const int m = row < M ? row : M - 1;
-      off[j] = (uint32_t)((int64_t)m * lda + chunk * 8);
+    is_w[j] = row >= 16 * MB;
+    if (row < 16 * MB) {
+      off[j] = (uint32_t)((int64_t)row_map(16 * MB * tile_m + row, M) * lda + chunk * 8);
     } else {
-      off[j] = (uint32_t)((int64_t)(tile_n * 16 + row - 32) * K + chunk * 8);
+      off[j] = (uint32_t)((int64_t)(tile_n * 16 * NB + row - 16 * MB) * K + chunk * 8);
     }
   }
   auto issue = [&](half_t* st, int k0) {
@@ -1007,15 +1031,15 @@ __global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restri
   };
 
   // Fragments of K slice s of a stage: lane (g, r) holds k = 16 s + 4 g ..
-  // + 3 of A row 16 w + r and of W row r; W is the MFMA A operand, so the
-  // lane accumulates C row 16 w + r at columns 4 g .. 4 g + 3 of the tile.
+  // + 3 of A row 16 wm + r and of W row 16 wn + r; W is the MFMA A operand, so the
+  // lane accumulates C row 16 wm + r at columns 16 wn + 4 g .. + 3 of the tile.
   half4_t fa[2][kSkBK / 16], fw[2][kSkBK / 16];
   auto read_frags = [&](const half_t* st, int set) {
 #pragma unroll
     for (int s = 0; s < kSkBK / 16; ++s) {
       const int chunk = 2 * s + (g >> 1), sub = 4 * (g & 1);
-      fa[set][s] = *reinterpret_cast<const half4_t*>(st + sk_offset(16 * wave + r, chunk) + sub);
-      fw[set][s] = *reinterpret_cast<const half4_t*>(st + sk_offset(32 + r, chunk) + sub);
+      fa[set][s] = *reinterpret_cast<const half4_t*>(st + sk_offset(16 * wm + r, chunk) + sub);
+      fw[set][s] = *reinterpret_cast<const half4_t*>(st + sk_offset(16 * MB + 16 * wn + r, chunk) + sub);
     }
   };
   float4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -1025,26 +1049,27 @@ __global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restri
   // vmcnt(N).
   const int nk = K / kSkBK;
   const int last_k0 = (nk - 1) * kSkBK;
-  // (the eight buffers as compile-time constants, in order)
+  // (the buffers as compile-time constants, in order)
   auto each_buffer = [&](auto&& f) {
-    f(ic<0>{}), f(ic<1>{}), f(ic<2>{}), f(ic<3>{}), f(ic<4>{}), f(ic<5>{}), f(ic<6>{}), f(ic<7>{});
+    f(ic<0>{}), f(ic<1>{}), f(ic<2>{}), f(ic<3>{});
+    if constexpr (NST > 4) f(ic<4>{}), f(ic<5>{}), f(ic<6>{}), f(ic<7>{});
   };
   each_buffer([&](auto b) { issue(stage(b), min(decltype(b)::value * kSkBK, last_k0)); });
-  wait_vmcnt<(kSkStages - 1) * kSkLoads>();  // stage 0 landed
+  wait_vmcnt<(NST - 1) * kSkLoads>();  // stage 0 landed
   stage_barrier();
   read_frags(stage(ic<0>{}), 0);
 
   // Step kt on buffer B: stage kt + 1 landed everywhere and every wave is
   // done with buffer B (its fragments were read a step earlier); B is
-  // refilled with stage kt + 8; the fragments of stage kt + 1 are read, and
+  // refilled with stage kt + NST; the fragments of stage kt + 1 are read, and
   // their LDS latency passes under the MFMA chain of stage kt, whose
   // fragments are already in registers.
   auto step = [&](auto b, int kt) {
     constexpr int B = decltype(b)::value;
-    wait_vmcnt<(kSkStages - 2) * kSkLoads>();
+    wait_vmcnt<(NST - 2) * kSkLoads>();
     stage_barrier();
-    issue(stage(b), min((kt + kSkStages) * kSkBK, last_k0));
-    read_frags(stage(ic<(B + 1) % kSkStages>{}), (B + 1) & 1);  // unused after the last step
+    issue(stage(b), min((kt + NST) * kSkBK, last_k0));
+    read_frags(stage(ic<(B + 1) % NST>{}), (B + 1) & 1);  // unused after the last step
     // (the scheduler would otherwise pull each MFMA up to the fragment read
     // it needs next and wait for that read inside the chain)
     __builtin_amdgcn_sched_barrier(0);
@@ -1054,15 +1079,15 @@ __global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restri
     __builtin_amdgcn_sched_barrier(0);
   };
   int kt = 0;
-  for (; kt + kSkStages <= nk; kt += kSkStages) each_buffer([&](auto b) { step(b, kt + decltype(b)::value); });
+  for (; kt + NST <= nk; kt += NST) each_buffer([&](auto b) { step(b, kt + decltype(b)::value); });
   each_buffer([&](auto b) {
     if (kt + decltype(b)::value < nk) step(b, kt + decltype(b)::value);
   });
   wait_vmcnt<0>();  // every DMA landed before the workgroup's LDS is released
 
-  const int row = 16 * wave + r;
+  const int row = 16 * (MB * tile_m + wm) + r;
   if (row < M) {
-    const int col = tile_n * 16 + 4 * g;
+    const int col = (tile_n * NB + wn) * 16 + 4 * g;
     half4_t v;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = epilogue<EPI>(acc[e], EPI != GD_EPI_NONE ? (float)bias[col + e] : 0.f);
@@ -1070,11 +1095,14 @@ __global__ __launch_bounds__(128) void gemm_skinny_kernel(const half_t* __restri
   }
 }
 
+template <int MB, int NB, int NST, class Rows>
 int launch_skinny(const half_t* A, const half_t* W, const half_t* bias, half_t* C, int M, int N, int K, int64_t lda,
-                  int64_t ldc, int epi, hipStream_t stream) {
-  const dim3 grid(N / 16), block(128);
+                  int64_t ldc, Rows rows, int epi, hipStream_t stream) {
+  const int tiles_m = (M + 16 * MB - 1) / (16 * MB);
+  const dim3 grid(tiles_m * (N / (16 * NB))), block(64 * MB * NB);
 #define GD_SKINNY(E) \
-  hipLaunchKernelGGL((gemm_skinny_kernel<E>), grid, block, 0, stream, A, W, bias, C, M, N, K, lda, ldc)
+  hipLaunchKernelGGL((gemm_skinny_kernel<MB, NB, NST, E, Rows>), grid, block, 0, stream, A, W, bias, C, M, N, K, lda, ldc, tiles_m, \
+                     rows)
   switch (epi) {
     case GD_EPI_NONE: GD_SKINNY(GD_EPI_NONE); break;
     case GD_EPI_BIAS: GD_SKINNY(GD_EPI_BIAS); break;
@@ -1171,12 +1199,17 @@ constexpr TileCost kTileCosts[] = {
     {256, 256, 8.44f, 16.34f, 7.79f},
 };
 
-// Index into kTileCosts of the cheapest tile for an M x N x K product.
-int cheapest_tile(int M, int N, int K, bool gelu, int64_t cus) {
+// Returned where a launch rule has no tile for a product.
+constexpr int kNoTile = 1;
+
+// Index into kTileCosts of the cheapest of its first `candidates` tiles for an
+// M x N x K product.
+int cheapest_tile(int M, int N, int K, bool gelu, int64_t cus,
+                  int candidates = (int)(sizeof kTileCosts / sizeof kTileCosts[0])) {
   int best = 0;
   double best_us = 1e30;
   const double kk = K / 1024.0;
-  for (int i = 0; i < (int)(sizeof kTileCosts / sizeof kTileCosts[0]); ++i) {
+  for (int i = 0; i < candidates; ++i) {
     const TileCost& t = kTileCosts[i];
     if (N % t.bn) continue;
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * (N / t.bn);
@@ -1202,22 +1235,43 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
   auto Bv = static_cast<const half_t*>(bias);
   auto Cm = static_cast<half_t*>(c);
   const int M = (int)m, N = (int)n, K = (int)k;
-  // Tile choice: 256-row tiles once there are enough rows to fill the chip,
-  // smaller tiles for short inputs (classifier head, short buckets).
-  if (a_rows) {
-    if (M >= 1024) return launch_tile<128, 128, true>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
-    return launch_tile<64, 128, true>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
-  }
   // The DMA tile kernels address A and W by 32-bit element offsets; larger
   // operands take the register-staged kernel (same accumulation order).
-  if ((int64_t)(M - 1) * lda + K >= (int64_t{1} << 31) || (int64_t)N * K >= (int64_t{1} << 31))
-    return launch_tile<128, 128, false>(A, Wt, Bv, Cm, M, N, K, lda, ldc, nullptr, 0, epilogue_kind, stream);
-  // At most 32 rows: 32 x 16 tiles, one MFMA chain per wave, eight stages in
-  // flight.
-  if (M <= 32 && N % 16 == 0 && K % kSkBK == 0)
-    return launch_skinny(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
-  if (M <= 4096 && N % 128 == 0 && K % 64 == 0) {
-    switch (cheapest_tile(M, N, K, epilogue_kind == GD_EPI_BIAS_GELU, gemm_cu_count())) {
+  const int64_t a_last = (a_rows ? a_row_count : m) - 1;
+  if (a_last * lda + K >= (int64_t{1} << 31) || (int64_t)N * K >= (int64_t{1} << 31)) {
+    if (a_rows) return launch_tile<true>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
+    return launch_tile<false>(A, Wt, Bv, Cm, M, N, K, lda, ldc, nullptr, 0, epilogue_kind, stream);
+  }
+  const int64_t cus = gemm_cu_count();
+  const bool gelu = epilogue_kind == GD_EPI_BIAS_GELU;
+  auto with_rows = [&](auto rows) -> int {
+    // Few rows: skinny tiles, 32 rows on 16 columns up to 32 rows, else the
+    // smaller of 32 x 32 and 64 x 32 that fits one round of workgroups (FFN-down
+    // at 64, 256, 300 and 512 rows 7.8, 8.1, 10.2 and 11.5 us against 15.4 to
+    // 15.7 on 64 x 64 tiles, QKV at 64 and 128 rows 4.4 and 5.2 against 6.4;
+    // in a second round they lose: QKV at 300 rows 9.7 against 6.9).
+    if (K % kSkBK == 0) {
+      if (M <= 32) return launch_skinny<2, 1, 8>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
+      if ((int64_t)((M + 31) / 32) * (N / 32) <= cus)
+        return launch_skinny<2, 2, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
+      if ((int64_t)((M + 63) / 64) * (N / 32) <= cus)
+        return launch_skinny<4, 2, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
+    }
+    return kNoTile;
+  };
+  if (a_rows) {
+    const GatheredRows rows{a_rows, (int)a_row_count};
+    const int st = with_rows(rows);
+    if (st != kNoTile) return st;
+    // Gathered rows (marker rows, at most a few thousand): the cheaper of two tiles.
+    if (cheapest_tile(M, N, K, gelu, cus, 2) == 0)
+      return launch_lds_tile<64, 64, 2, 64, 4, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream, rows);
+    return launch_lds_tile<128, 128, 2, 64, 2, 8>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream, rows);
+  }
+  if (const int st = with_rows(PlainRows{}); st != kNoTile) return st;
+  // (N is a multiple of 128 and K of 64 from here on: both callers check)
+  if (M <= 4096) {
+    switch (cheapest_tile(M, N, K, gelu, cus)) {
       case 0: return launch_lds_tile<64, 64, 2, 64, 4, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
       case 1: return launch_lds_tile<128, 128, 2, 64, 2>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
       case 2:
@@ -1229,7 +1283,7 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
       default: return launch_lds_tile<256, 256, 2, 64, 2>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
     }
   }
-  if (M >= 2048 && N % 256 == 0) {
+  if (N % 256 == 0) {
     // Whole rounds of 256 x 256 tiles (one tile per CU) over the first rows
     // and, when the rows left over fit one round of 128 x 128 tiles and would
     // cost the 256 x 256 launch a further round, those in a second launch: a
@@ -1239,7 +1293,6 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
     // (N = 3072 on 32,768 rows: 1,536 tiles, six rounds either way) the
     // second launch only adds its own ramp (212 against 199 us).  Every
     // kernel accumulates in the same order and reads the GELU table.
-    const int64_t cus = gemm_cu_count();
     const int64_t m_tiles_round = cus / (N / 256);
     // GELU (FFN-up) on up to 320 rows per tile row: one round of 320 x 256
     // tiles where 256 x 256 tiles would need a second (FFN-up at 4,896 rows).
@@ -1256,14 +1309,13 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
                                                  lda, ldc, epilogue_kind, stream);
     }
   }
-  if (M >= 2048) {
+  {
     // 256-row tiles: 256 x 256 (two 64-deep stages, 128 KiB of LDS), 256 x 192
     // (two stages, 112 KiB) or 256 x 128 (three stages, 144 KiB), whichever
     // finishes first: rounds of one tile per CU, each costing the tile's
     // measured time per round relative to a 256 x 128 tile (1.5, 1.35, 1; K =
     // 1024 and 4096 alike, from a sweep of every tile kernel over 4,896 to
     // 32,768 rows).  Ties keep the larger tile.
-    const int64_t cus = gemm_cu_count();
     auto rounds = [&](int bm, int bn) { return (double)((((M + bm - 1) / bm) * (N / bn) + cus - 1) / cus); };
     // One round of 160 x 128 tiles (three stages, 108 KiB) where it fits:
     // out-proj and FFN-down on up to 5,120 packed rows run 248 tiles instead
@@ -1300,14 +1352,6 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
     if (bm == 192) return launch_lds_tile<192, 128, 2, 64, 3>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
     return launch_lds_tile<256, 128, 4, 64, 3>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
   }
-  // Widths that are a multiple of 64 but not of 128: 64 x 64 DMA-pipelined
-  // tiles of four waves with four 64-deep stages in flight (the
-  // register-staged kernel keeps one K step in flight, which left a 160-row
-  // K = 4096 product waiting on global latency for 55 us).
-  if (N % 64 == 0 && K % 64 == 0)
-    return launch_lds_tile<64, 64, 2, 64, 4, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream);
-  if (M >= 1024) return launch_tile<128, 128, false>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
-  return launch_tile<64, 128, false>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
 }
 
 

@@ -135,6 +135,30 @@ def test_embedding_layer_norm():
 # ---------------------------------------------------------------------------
 # linear (DeBERTa.swift:60-92, 421, 437)
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("n,k,epilogue", [(1024, 4096, "bias"), (3072, 1024, "bias"), (4096, 1024, "gelu"),
+                                          (2048, 1024, "relu"), (384, 192, "bias")])
+def test_linear_few_rows_and_gathered_rows(n, k, epilogue):
+    """Every row of a product has the bits that the 8,192-row product gives
+    it, at the row counts where the skinny tiles change (32 rows, one round of
+    32-row and of 64-row tiles, K = 192 without them), and where the rows are
+    gathered (any order, repeats; indices outside the operand read the nearest
+    row, as the clamp states)."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + k)
+    x = torch.randn((8192, k), generator=g, device="cuda").half()
+    w = (0.02 * torch.randn((n, k), generator=g, device="cuda")).half()
+    b = torch.randn((n,), generator=g, device="cuda").half()
+    full = fk().linear(x, w, b, epilogue)
+    per_round = 256 // (n // 32)
+    for m in sorted({1, 31, 32, 33, 63, 65, 300, 32 * per_round, 32 * per_round + 1, 64 * per_round,
+                     64 * per_round + 1, 1025}):
+        assert torch.equal(fk().linear(x[:m], w, b, epilogue), full[:m]), m
+        rows = torch.randint(0, 8192, (m,), generator=g, device="cuda", dtype=torch.int32)
+        assert torch.equal(fk().linear(x, w, b, epilogue, rows=rows), full[rows.long()]), m
+    rows = torch.tensor([-5, 0, 8191, 9000] * 20, dtype=torch.int32, device="cuda")
+    assert torch.equal(fk().linear(x, w, b, epilogue, rows=rows), full[rows.long().clamp(0, 8191)])
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 128, 64), (65, 256, 128), (300, 1024, 1024), (1000, 384, 192),
                                    (160, 1024, 4096), (160, 4096, 1024), (37, 2048, 1024),
                                    (4096, 1024, 256), (4896, 1024, 4096),  # one round of 160x128 tiles
