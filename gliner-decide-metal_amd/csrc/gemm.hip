@@ -345,13 +345,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __re
   static_assert(EPI != GD_EPI_BIAS_GELU || GELU_TABLE || NSTAGE * RPA >= BM, "GELU epilogue staging");
   // Tiles whose stage buffers hold 128 KiB (and whose GELU values all fit
   // the registers before C is staged) read the full 65,536-entry table:
-  // the stages are then one array, the table lands in it after the K loop.
+  // the stages are then one array, the table lands in it at the K loop's end.
   // The 320-row tiles stage C one wave row (160 rows) per pass in that array
   // (FFN-up at 4,896 rows 52.4-53.3 -> 51.4-52.7 us against the compact table
   // DMA'd under the last K step; the packed step +1.3%, its FFN-down reading
   // the plainly stored output).
   constexpr int RPF = NSTAGE * STAGE / BN / WM * WM;  // whole wave rows that the joined stages hold
   constexpr bool FULLTAB = GELU_TABLE && NSTAGE * STAGE >= 65536 && (BM == 320 ? RPF >= WM : RPA % WM == 0);
+  constexpr bool TABTAIL = FULLTAB && NSTAGE == 2;        // the table comes under the last two K steps
   constexpr int RPP = FULLTAB && BM == 320 ? RPF : RPA;  // C rows per pass of the GELU epilogue
   constexpr int TAB1 = NSTAGE == 2 || kGeluEntries <= STAGE ? kGeluEntries : STAGE;  // entries in st1
   constexpr int kA = FULLTAB ? 16 : 1024;  // alignment of the separate buffers (unused with FULLTAB)
@@ -498,21 +499,79 @@ __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __re
     mma((S - 1) & 1);
     interleave();
   };
-  // Whole groups of NSTAGE steps run branch-free (a branch between steps
-  // would merge waitcnt states and cost a full vmcnt(0) drain); the
-  // remaining nk % NSTAGE steps follow the loop.
-  int kt = 0;
-  for (; kt + NSTAGE <= nk; kt += NSTAGE) {
-    step(ic<0>{}, kt);
-    step(ic<1>{}, kt + 1);
-    if constexpr (NSTAGE > 2) step(ic<2>{}, kt + 2);
-    if constexpr (NSTAGE > 3) step(ic<3>{}, kt + 3);
-    if constexpr (NSTAGE > 4) step(ic<4>{}, kt + 4);
+  if constexpr (TABTAIL) {
+    // Two-stage tiles that read the full GELU table bring it under the last K steps: those
+    // have nothing left to fetch, and each part of the table goes into the
+    // buffer that has just become free (4,096 columns on 32,768, 8,192 and 4,896
+    // rows 307 -> 296, 85.7 -> 83.8 and 49.2 -> 47.8 us against a table brought
+    // after the loop).  The bias epilogues keep the loop below: without a table
+    // the tail gained nothing, and K = 4096 lost 5% to it.
+    auto issue_table = [&](auto b) {
+      constexpr int FROM = decltype(b)::value * STAGE, TO = FROM + STAGE < 65536 ? FROM + STAGE : 65536;
+      for (int j = FROM / 512 + wave; j < TO / 512; j += NW)
+        load_lds16(g_gelu_full + j * 512 + lane * 8, stall + j * 512);
+    };
+    auto tail = [&](auto b, auto i) {  // the last step but one (I = 0), on buffer b, and the last
+      constexpr int B = decltype(b)::value, I = decltype(i)::value;
+#pragma unroll
+      for (int s = 0; s + 1 < S; ++s) {
+        read_frags(stage(b), s + 1, (s + 1) & 1);
+        mma(s & 1);
+        interleave();
+      }
+      if constexpr (I == 0) {
+        wait_vmcnt<0>();
+        stage_barrier();
+        issue_table(b);
+        read_frags(stage(ic<1 - B>{}), 0, 0);
+        mma((S - 1) & 1);
+        interleave();
+      } else {
+        stage_barrier();  // every wave's fragments are in registers
+        issue_table(b);
+        mma((S - 1) & 1);
+      }
+    };
+    auto rest = [&](auto r, int kt) {
+      constexpr int R = decltype(r)::value;
+      if constexpr (R > 0) step(ic<0>{}, kt);
+      tail(ic<R>{}, ic<0>{});
+      tail(ic<1 - R>{}, ic<1>{});
+    };
+    // (each remainder is a straight path of its own: a branch between steps
+    // would merge waitcnt states and cost a full vmcnt(0) drain)
+    if (nk >= 2) {
+      int kt = 0;
+      for (; kt + 2 <= nk - 2; kt += 2) {
+        step(ic<0>{}, kt);
+        step(ic<1>{}, kt + 1);
+      }
+      const int r = nk - 2 - kt;
+      if (r == 0) rest(ic<0>{}, kt);
+      if (r == 1) rest(ic<1>{}, kt);
+    } else {
+      step(ic<0>{}, 0);
+      wait_vmcnt<0>();
+      __syncthreads();
+      issue_table(ic<0>{}), issue_table(ic<1>{});
+    }
+  } else {
+    // Whole groups of NSTAGE steps run branch-free (a branch between steps
+    // would merge waitcnt states and cost a full vmcnt(0) drain); the
+    // remaining nk % NSTAGE steps follow the loop.
+    int kt = 0;
+    for (; kt + NSTAGE <= nk; kt += NSTAGE) {
+      step(ic<0>{}, kt);
+      step(ic<1>{}, kt + 1);
+      if constexpr (NSTAGE > 2) step(ic<2>{}, kt + 2);
+      if constexpr (NSTAGE > 3) step(ic<3>{}, kt + 3);
+      if constexpr (NSTAGE > 4) step(ic<4>{}, kt + 4);
+    }
+    if (kt < nk) step(ic<0>{}, kt);
+    if constexpr (NSTAGE > 2) if (kt + 1 < nk) step(ic<1>{}, kt + 1);
+    if constexpr (NSTAGE > 3) if (kt + 2 < nk) step(ic<2>{}, kt + 2);
+    if constexpr (NSTAGE > 4) if (kt + 3 < nk) step(ic<3>{}, kt + 3);
   }
-  if (kt < nk) step(ic<0>{}, kt);
-  if constexpr (NSTAGE > 2) if (kt + 1 < nk) step(ic<1>{}, kt + 1);
-  if constexpr (NSTAGE > 3) if (kt + 2 < nk) step(ic<2>{}, kt + 2);
-  if constexpr (NSTAGE > 4) if (kt + 3 < nk) step(ic<3>{}, kt + 3);
   wait_vmcnt<0>();  // every DMA (the GELU table's too) landed
   __syncthreads();  // all waves done reading the stage buffers
 
@@ -562,13 +621,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __re
     const half_t* tab2 = stage(ic<2 % NSTAGE>{});
     constexpr uint32_t kSplit = TAB1;
     half_t* const cst = FULLTAB ? stall : st0;
-    if constexpr (FULLTAB) {
+    if constexpr (FULLTAB && !TABTAIL) {
       // the full table by DMA into the stage buffers (all read: the K loop's
       // last barrier), wave w taking 1 KiB blocks w, w + NW, ...
       for (int j = wave; j < 65536 / 512; j += NW) load_lds16(g_gelu_full + j * 512 + lane * 8, stall + j * 512);
       wait_vmcnt<0>();
       __syncthreads();
-    } else {
+    } else if constexpr (!FULLTAB) {
       // All of this thread's table pieces are loaded before any is stored,
       // so the L2 latency is paid once.
       constexpr int kPieces = kGeluEntries / 8;
@@ -897,7 +956,7 @@ int launch_lds_split160(const half_t* A, const half_t* W, const half_t* bias, ha
 }
 
 // 320 x 256 tiles (two 64-deep stages, 144 KiB, the full GELU table in them
-// after the K loop), GELU epilogue only: one round over up to 320 rows per
+// from the last K steps on), GELU epilogue only: one round over up to 320 rows per
 // tile row where 256-row tiles need a second.
 int launch_lds_tile_gelu320(const half_t* A, const half_t* W, const half_t* bias, half_t* C, int M, int N, int K,
                             int64_t lda, int64_t ldc, hipStream_t stream) {

@@ -135,6 +135,22 @@ def test_embedding_layer_norm():
 # ---------------------------------------------------------------------------
 # linear (DeBERTa.swift:60-92, 421, 437)
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("m", [4896, 8192])
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320])
+def test_linear_gelu_table_under_the_last_k_steps(m, k):
+    """The tiles that bring the GELU table under their last two K steps (320 x
+    256 at 4,896 rows, 256 x 256 at 8,192), at one, two, odd and even counts
+    of K steps: every row has the bits of the small tiles' product."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + k)
+    x = torch.randn((m, k), generator=g, device="cuda").half()
+    w = (0.1 * torch.randn((4096, k), generator=g, device="cuda")).half()
+    b = torch.randn((4096,), generator=g, device="cuda").half()
+    full = fk().linear(x, w, b, "gelu")
+    for lo in (0, 317, m - 300):
+        assert torch.equal(fk().linear(x[lo:lo + 300].contiguous(), w, b, "gelu"), full[lo:lo + 300]), lo
+
+
 @pytest.mark.parametrize("n,k,epilogue", [(1024, 4096, "bias"), (3072, 1024, "bias"), (4096, 1024, "gelu"),
                                           (2048, 1024, "relu"), (384, 192, "bias")])
 def test_linear_few_rows_and_gathered_rows(n, k, epilogue):
