@@ -26,8 +26,11 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(stream: torch.cuda.Stream | None = None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    # The handle alone: a torch.cuda.Stream object costs more than the rest of
+    # a small call's arguments.
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def as_f16(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -35,7 +38,7 @@ def as_f16(t: torch.Tensor, name: str) -> torch.Tensor:
         raise ValueError(f"{name} must be on the GPU")
     if t.dtype != torch.float16:
         raise TypeError(f"{name} must be float16 (got {t.dtype})")
-    return t.contiguous()
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def as_i32(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -43,4 +46,6 @@ def as_i32(t: torch.Tensor, name: str) -> torch.Tensor:
         raise ValueError(f"{name} must be on the GPU")
     if t.dtype not in (torch.int32, torch.int64):
         raise TypeError(f"{name} must be an integer tensor (got {t.dtype})")
-    return t.to(torch.int32).contiguous()
+    if t.dtype != torch.int32:
+        t = t.to(torch.int32)
+    return t if t.is_contiguous() else t.contiguous()

@@ -31,9 +31,25 @@ def _indices(c2p_indices, p2c_indices, H: int, L: int):
         return None, None
     if c2p_indices is None or p2c_indices is None:
         raise N.GlinerDecideError(N.GD_ERR_INVALID_ARGUMENT, "give both index tensors, or neither")
-    c2p = as_i32(c2p_indices, "c2p_indices").expand(1, H, L, L).reshape(H, L, L).contiguous()
-    p2c = as_i32(p2c_indices, "p2c_indices").expand(1, H, L, L).reshape(H, L, L).contiguous()
-    return c2p, p2c
+    return _index_tensor(c2p_indices, "c2p_indices", H, L), _index_tensor(p2c_indices, "p2c_indices", H, L)
+
+
+def _index_tensor(t: torch.Tensor, name: str, H: int, L: int) -> torch.Tensor:
+    t = as_i32(t, name)
+    return t if t.shape == (H, L, L) else t.expand(1, H, L, L).reshape(H, L, L).contiguous()
+
+
+def _shaped(t: torch.Tensor, name: str, *shape: int) -> torch.Tensor:
+    t = as_f16(t, name)
+    return t if t.shape == shape else t.reshape(shape).contiguous()
+
+
+_OUTPUTS = {"probs": N.GD_ATTN_OUT_PROBS, "context": N.GD_ATTN_OUT_CONTEXT, "bias": N.GD_ATTN_OUT_BIAS}
+_SCORES = {"default": N.GD_ATTN_SCORE_DEFAULT, "explicit": N.GD_ATTN_SCORE_EXPLICIT,
+           "kernel_bias": N.GD_ATTN_SCORE_KERNEL_BIAS, "kernel_bias_explicit": N.GD_ATTN_SCORE_KERNEL_BIAS_EXPLICIT,
+           "fused": N.GD_ATTN_SCORE_FUSED}
+_MASKS = {"attention": N.GD_MASK_ATTENTION, "additive": N.GD_MASK_ADDITIVE}
+_EPILOGUES = {"none": N.GD_EPI_NONE, "bias": N.GD_EPI_BIAS, "gelu": N.GD_EPI_BIAS_GELU, "relu": N.GD_EPI_BIAS_RELU}
 
 
 class FusedKernels:
@@ -81,9 +97,9 @@ class FusedKernels:
             raise N.GlinerDecideError(N.GD_ERR_SHAPE, "q/k must both be [B, H, L, D]")
         H, L = heads, sequence_length
         c2p, p2c = _indices(c2p_indices, p2c_indices, H, L)
-        pk = as_f16(position_key, "position_key").reshape(H, position_count, head_dimension).contiguous()
-        pq = as_f16(position_query, "position_query").reshape(H, position_count, head_dimension).contiguous()
-        km = as_f16(key_mask, "key_mask").reshape(batch, L).contiguous()
+        pk = _shaped(position_key, "position_key", H, position_count, head_dimension)
+        pq = _shaped(position_query, "position_query", H, position_count, head_dimension)
+        km = _shaped(key_mask, "key_mask", batch, L)
         out = torch.empty((batch, H, L, L), dtype=torch.float16, device=q.device)
         N.check(self._lib.gd_relative_bias(ptr(q), ptr(k), ptr(pk), ptr(pq), ptr(c2p), ptr(p2c), ptr(km),
                                            float(scale), batch, H, L, head_dimension, position_count, ptr(out),
@@ -105,9 +121,9 @@ class FusedKernels:
             raise N.GlinerDecideError(N.GD_ERR_SHAPE, "queries shape does not match the given dimensions")
         H, L = heads, sequence_length
         c2p, p2c = _indices(c2p_indices, p2c_indices, H, L)
-        pk = as_f16(position_key, "position_key").reshape(H, position_count, head_dimension).contiguous()
-        pq = as_f16(position_query, "position_query").reshape(H, position_count, head_dimension).contiguous()
-        km = as_f16(key_mask, "key_mask").reshape(batch, L).contiguous()
+        pk = _shaped(position_key, "position_key", H, position_count, head_dimension)
+        pq = _shaped(position_query, "position_query", H, position_count, head_dimension)
+        km = _shaped(key_mask, "key_mask", batch, L)
         out = torch.empty((batch, L, H, head_dimension), dtype=torch.float16, device=q.device)
         N.check(self._lib.gd_fused_attention(ptr(q), ptr(k), ptr(v), ptr(pk), ptr(pq), ptr(c2p), ptr(p2c), ptr(km),
                                              float(scale), batch, H, L, head_dimension, position_count, ptr(out),
@@ -138,12 +154,8 @@ class FusedKernels:
             if t.dim() != 3 or t.shape[0] != H or t.shape[2] != D or t.stride(2) != 1 or t.dtype != torch.float16:
                 raise N.GlinerDecideError(N.GD_ERR_SHAPE, f"{name} must be a [H, P, D] fp16 view with contiguous D")
         P = position_key.shape[1]
-        mask = as_f16(mask, "mask").reshape(B, L).contiguous()
-        kind = {"probs": N.GD_ATTN_OUT_PROBS, "context": N.GD_ATTN_OUT_CONTEXT, "bias": N.GD_ATTN_OUT_BIAS}[output]
-        sc = {"default": N.GD_ATTN_SCORE_DEFAULT, "explicit": N.GD_ATTN_SCORE_EXPLICIT,
-              "kernel_bias": N.GD_ATTN_SCORE_KERNEL_BIAS, "kernel_bias_explicit": N.GD_ATTN_SCORE_KERNEL_BIAS_EXPLICIT,
-              "fused": N.GD_ATTN_SCORE_FUSED}[score]
-        mk = {"attention": N.GD_MASK_ATTENTION, "additive": N.GD_MASK_ADDITIVE}[mask_kind]
+        mask = _shaped(mask, "mask", B, L)
+        kind, sc, mk = _OUTPUTS[output], _SCORES[score], _MASKS[mask_kind]
         if out is None:
             shape = (B, L, H * D) if kind == N.GD_ATTN_OUT_CONTEXT else (B, H, L, L)
             out = torch.empty(shape, dtype=torch.float16, device=q.device)
@@ -180,16 +192,15 @@ class FusedKernels:
         N_, K = _dims(w, 2, "weight")
         if x.shape[-1] != K:
             raise N.GlinerDecideError(N.GD_ERR_SHAPE, f"x last dim {x.shape[-1]} != weight in-features {K}")
-        x2 = x.reshape(-1, K)
+        x2 = x if x.dim() == 2 else x.reshape(-1, K)
         if rows is not None:
-            rows = as_i32(rows, "rows").reshape(-1)
+            rows = as_i32(rows, "rows")
             M = rows.numel()
             lead = (M,)
         else:
             M = x2.shape[0]
             lead = tuple(x.shape[:-1])
-        epi = {"none": N.GD_EPI_NONE, "bias": N.GD_EPI_BIAS, "gelu": N.GD_EPI_BIAS_GELU,
-               "relu": N.GD_EPI_BIAS_RELU}[epilogue]
+        epi = _EPILOGUES[epilogue]
         b = as_f16(bias, "bias") if bias is not None else None
         out = torch.empty(lead + (N_,), dtype=torch.float16, device=x.device)
         N.check(self._lib.gd_linear(ptr(x2), ptr(w), ptr(b), ptr(out), M, N_, K, K, N_, ptr(rows), x2.shape[0], epi,
