@@ -729,8 +729,8 @@ def test_general_index_kernels_any_length(L, P, H, B, relative):
     if relative:
         rel = np.arange(L)[:, None] - np.arange(L)[None, :]
         idx = np.clip(O.relative_bucket(rel) + 256, 0, P - 1).astype(np.int32)
-        c2p = np.ascontiguousarray(np.broadcast_to(idx, (H, L, L)))
-        p2c = np.ascontiguousarray(np.broadcast_to(idx.T, (H, L, L)))
+        c2p = np.broadcast_to(idx, (H, L, L)).copy()
+        p2c = np.broadcast_to(idx.T, (H, L, L)).copy()
     else:
         c2p = r.integers(0, P, size=(H, L, L)).astype(np.int32)
         p2c = r.integers(0, P, size=(H, L, L)).astype(np.int32)
