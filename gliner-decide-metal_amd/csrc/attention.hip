@@ -693,9 +693,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto c_of = [](uint32_t cp) { return (int)(cp & 0xFFFFu); };
   auto p_of = [](uint32_t cp) { return (int)(cp >> 16); };
 
-  // running max (per query row, the same in the row's four lanes), this
-  // lane's part of the row sum, and O^T (lane: query lc, d 16 dt + 4 g + i)
-  float m_run = -65504.f, l_run = 0.f;
+  // running max (per query row, the same in the row's four lanes) and its
+  // rounded product with log2 e, this lane's part of the row sum, and O^T
+  // (lane: query lc, d 16 dt + 4 g + i)
+  constexpr float kLog2e = 1.4426950408889634f;
+  float m_run = -65504.f, m_l2 = m_run * kLog2e, l_run = 0.f;
   float4_t o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = (float4_t){0.f, 0.f, 0.f, 0.f};
@@ -799,7 +801,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int j = 0; j < 4; ++j) cp[kb][j] = cpn[kb][j];
 
     // ---- online softmax over this key block, then P . V ----
-    constexpr float kLog2e = 1.4426950408889634f;
     float bmax = m_run;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
@@ -811,11 +812,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         bmax = fmaxf(bmax, sc);
       }
     bmax = rows_max(bmax);
-    // exp(s - m) = 2^(s log2e - m log2e); the rounding of m log2e scales a
-    // whole row alike and cancels in the normalisation.
-    const float alpha = __builtin_amdgcn_exp2f(m_run * kLog2e - bmax * kLog2e);
-    m_run = bmax;
-    const float m_l2 = bmax * kLog2e;
+    // exp(s - m) = 2^(s log2e - m log2e), m log2e rounded once per block: the
+    // rounding scales a row's weights alike, and carries from block to block in
+    // m_l2, so that it cancels in the normalisation and alpha is 1 where the
+    // max stays.  (The empty asm keeps the product out of alpha's subtraction:
+    // in an fma with it, alpha would be 2^residual, 0.9985 at the max of a row
+    // whose keys are all masked.)
+    float next_l2 = bmax * kLog2e;
+    asm("" : "+v"(next_l2));
+    const float alpha = __builtin_amdgcn_exp2f(m_l2 - next_l2);
+    m_run = bmax, m_l2 = next_l2;
     l_run *= alpha;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;

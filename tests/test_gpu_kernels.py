@@ -753,6 +753,33 @@ def test_general_index_kernels_any_length(L, P, H, B, relative):
     assert np.max(np.abs(got - want)) <= 2e-3  # one fp16 rounding of values below 4
 
 
+@pytest.mark.parametrize("L", [65, 200, 256, 333, 500, 512])
+def test_fused_attention_all_masked_row_is_the_mean_of_v(L):
+    """With every key masked each weight is exp(-65504 - -65504) / L: the
+    output is the mean of V, over any number of key blocks.  Half of V's
+    columns are 1 in the first 64 keys and -1 in the last 64, which a scale
+    between key blocks would show.  Bound: the weights are equal, so what is
+    left is the fp32 sums' rounding (at most L + 4 of 2^-24 of mean |V|: L
+    terms, the row sum's reciprocal and two products) and half an fp16 ulp."""
+    B, H, P = 2, 2, 512
+    r = np.random.default_rng(2100 + L)
+    q, k, v = (r.standard_normal((B, H, L, 64)).astype(np.float16) for _ in range(3))
+    pkh, pqh = (r.standard_normal((H, P, 64)).astype(np.float16) for _ in range(2))
+    v[..., :32] = 0
+    v[:, :, :64, :32] += 1
+    v[:, :, -64:, :32] -= 1
+    idx = np.clip(O.relative_bucket(np.arange(L)[:, None] - np.arange(L)[None, :]) + 256, 0, P - 1).astype(np.int32)
+    c2p = np.broadcast_to(idx, (H, L, L)).copy()
+    p2c = np.broadcast_to(idx.T, (H, L, L)).copy()
+    key_mask = np.full((B, L), -65504.0, np.float16)
+    got = host(fk().fused_attention(*(dev(a) for a in (q, k, v, pkh, pqh, c2p, p2c, key_mask)), O.scale_f32(64), B, H,
+                                    L, 64, P))
+    v64 = v.astype(np.float64)
+    want = np.broadcast_to(v64.mean(axis=2)[:, None], got.shape)
+    bound = 0.5 * ulp16(want) + (L + 4) * 2.0 ** -24 * np.abs(v64).mean(axis=2)[:, None]
+    assert np.all(np.abs(got - want) <= bound), (np.abs(got - want) - bound).max()
+
+
 def test_general_index_kernels_clamp_out_of_range_indices():
     """Indices outside [0, P) read the nearest table row (the per-query
     kernels' rule, kept by the matrix-core kernels)."""
