@@ -482,14 +482,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
 //
 // Scores (masked keys -65504, keys past L -inf) feed an online softmax per
 // query row (running max seeded at -65504, the reference's seed), and P . V
-// runs on the matrix cores with P split into fp16 hi + lo (V rows in LDS, read
-// transposed by ds_read_b64_tr_b16); the output row is divided by the row's
-// sum at the end.  The next key block's windows, K and V rows come by DMA during
-// the softmax and P . V, its indices a block earlier; two barriers per block.
+// runs on the matrix cores with the fp32 weights split into fp16 parts (V rows
+// in LDS, read transposed by ds_read_b64_tr_b16); the output row is divided by
+// the row's sum at the end.  EXACT splits a weight into three parts that hold
+// its 24 bits: error against 64 bits beyond the output's rounding, in 2^-24 of
+// the sum of |w v|, over lengths 3 to 511 and normal, sharp (4 q), flat and
+// cancelling inputs: at most 25, the per-query kernel's 55.  Two parts (22 bits,
+// a floor of 2^-25 of the row's largest weight) reach 1,200 on sharp rows.
+//
+// The next key block's windows, K and V rows come by DMA during the softmax and
+// P . V, its indices a block earlier; two barriers per block.
 // Bound by the block's chain of LDS round trips with two waves per SIMD (79 KB
-// of LDS, 240 VGPRs).  B = 8, H = 16, L = 200: 24.8 us (the per-query kernel,
-// which served every length that is no multiple of 16, 495 us); B = 32, L =
-// 256: 88 us (64-row windows, a gather per window: 97 us).
+// of LDS, 240 and 248 VGPRs).  B = 8, H = 16, L = 200 (EXACT): 27.5 us (two
+// parts 25.5, P . V in fp32 products 33.6, the per-query kernel 495); B = 32,
+// L = 256: 90 us (64-row windows, a gather per window: 97 us).
 // ---------------------------------------------------------------------------
 constexpr int kGenWin = 128;  // table rows per window
 
@@ -503,8 +509,9 @@ __device__ __attribute__((aligned(16))) const half_t g_zero_row[64] = {};
 __device__ __forceinline__ int gen_swz(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
 // VEC: L is a multiple of 4, so the c2p indices and the mask of four
-// consecutive keys are one aligned load.
-template <bool VEC>
+// consecutive keys are one aligned load.  EXACT: P . V takes all 24 bits of
+// the weights.
+template <bool VEC, bool EXACT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void fused_attention_mfma_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v,
     const half_t* __restrict__ pos_key, const half_t* __restrict__ pos_query, const int32_t* __restrict__ c2p_idx,
@@ -693,11 +700,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto c_of = [](uint32_t cp) { return (int)(cp & 0xFFFFu); };
   auto p_of = [](uint32_t cp) { return (int)(cp >> 16); };
 
-  // running max (per query row, the same in the row's four lanes) and its
-  // rounded product with log2 e, this lane's part of the row sum, and O^T
-  // (lane: query lc, d 16 dt + 4 g + i)
+  // Weights are exp(s - m) = 2^(s log2e - log_max(m)), with m log2e rounded
+  // once per block (never part of an fma): the rounding scales a row's weights
+  // alike, and the rounded value is what carries from block to block, so that
+  // it cancels in the normalisation and the rescale is 1 where the max stays.
   constexpr float kLog2e = 1.4426950408889634f;
-  float m_run = -65504.f, m_l2 = m_run * kLog2e, l_run = 0.f;
+  auto log_max = [](float m) {
+#pragma clang fp contract(off)
+    return m * kLog2e;
+  };
+  // With EXACT, P . V takes weights times 2^15: the largest still fits fp16,
+  // and fp16 parts of small ones keep 15 more bits above the subnormal floor.
+  constexpr float kScaleP = EXACT ? 32768.f : 1.f;
+  // running max (per query row, the same in the row's four lanes), its
+  // log_max, this lane's part of the row sum, and O^T (lane: query lc, d 16 dt
+  // + 4 g + i)
+  float m_run = -65504.f, m_l2 = log_max(m_run), l_run = 0.f;
   float4_t o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = (float4_t){0.f, 0.f, 0.f, 0.f};
@@ -812,14 +830,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         bmax = fmaxf(bmax, sc);
       }
     bmax = rows_max(bmax);
-    // exp(s - m) = 2^(s log2e - m log2e), m log2e rounded once per block: the
-    // rounding scales a row's weights alike, and carries from block to block in
-    // m_l2, so that it cancels in the normalisation and alpha is 1 where the
-    // max stays.  (The empty asm keeps the product out of alpha's subtraction:
-    // in an fma with it, alpha would be 2^residual, 0.9985 at the max of a row
-    // whose keys are all masked.)
-    float next_l2 = bmax * kLog2e;
-    asm("" : "+v"(next_l2));
+    const float next_l2 = log_max(bmax);
     const float alpha = __builtin_amdgcn_exp2f(m_l2 - next_l2);
     m_run = bmax, m_l2 = next_l2;
     l_run *= alpha;
@@ -830,7 +841,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float e = __builtin_amdgcn_exp2f(fmaf(acc[kb][j], kLog2e, -m_l2));
-        acc[kb][j] = e;
+        acc[kb][j] = e * kScaleP;
         l_run += e;
       }
     {
@@ -846,40 +857,105 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int tr_sw = (2 * g + (lc >> 3)) & 7;
       const int tr_lane = (4 * g + (lc >> 2)) * 64 + 4 * (lc & 1);
       const int tr_c = (lc >> 1) & 1;
+      auto v_tile = [&](int T, int dt) -> half4_t {  // V[16 T + 4 g + i][16 dt + lc]
+        gen_lds_half_t* const a = rows3 + 16 * T * 64 + tr_lane + (((2 * dt + tr_c) ^ tr_sw) << 3);
+        return __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)a));
+      };
+      // Two tiles' V fragments against parts of P (registers 4 u + i of a
+      // fragment: key 16 (T + u) + 4 g + i).
+      auto v_frag = [&](int T, int dt) -> half8_t {
+        const half4_t h0 = v_tile(T, dt), h1 = v_tile(T + 1, dt);
+        half8_t vb;
 #pragma unroll
-      for (int T = 0; T < KB; T += 2) {
-        half8_t pa, pl;
+        for (int i = 0; i < 4; ++i) {
+          vb[i] = h0[i];
+          vb[4 + i] = h1[i];
+        }
+        return vb;
+      };
+      if constexpr (!EXACT) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int T = 0; T < KB; T += 2) {
+          half8_t pa, pl;
 #pragma unroll
-          for (int i = 0; i < 4; i += 2) {
-            const float x0 = acc[T + u][i], x1 = acc[T + u][i + 1];
-            const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-            pa[4 * u + i] = hi[0];
-            pa[4 * u + i + 1] = hi[1];
-            pl[4 * u + i] = (half_t)(x0 - (float)hi[0]);
-            pl[4 * u + i + 1] = (half_t)(x1 - (float)hi[1]);
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+              const float x0 = acc[T + u][i], x1 = acc[T + u][i + 1];
+              const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+              pa[4 * u + i] = hi[0];
+              pa[4 * u + i + 1] = hi[1];
+              pl[4 * u + i] = (half_t)(x0 - (float)hi[0]);
+              pl[4 * u + i + 1] = (half_t)(x1 - (float)hi[1]);
+            }
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) {
+            const half8_t vb = v_frag(T, dt);
+            o[dt] = mfma16x16x32(vb, pa, o[dt]);
+            o[dt] = mfma16x16x32(vb, pl, o[dt]);
           }
+        }
+      } else {
+        // All 24 bits of a weight x: hi + (mid + low) 2^-10 in fp16, exact for
+        // weights from 2^-25 of the row's largest on, below that to 2^-49 of
+        // it (512 of them on V = 65504: one subnormal step of the output).
+        float4_t before[4], rest[4];
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-          const gen_lds_half_t* a = rows3 + 16 * T * 64 + tr_lane + (((2 * dt + tr_c) ^ tr_sw) << 3);
-          const gen_short4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)a);
-          const gen_short4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gen_lds_short4_t*)(a + 16 * 64));
-          const half4_t h0 = __builtin_bit_cast(half4_t, v0), h1 = __builtin_bit_cast(half4_t, v1);
-          half8_t vb;
+        for (int dt = 0; dt < 4; ++dt) before[dt] = o[dt], rest[dt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int T = 0; T < KB; T += 2) {
+          half8_t pa, pm, pl;
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+              const float x0 = acc[T + u][i], x1 = acc[T + u][i + 1];
+              const half2_t hi = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+              const float r0 = (x0 - (float)hi[0]) * 1024.f, r1 = (x1 - (float)hi[1]) * 1024.f;
+              const half2_t mid = __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(r0, r1));
+              const half2_t low = __builtin_bit_cast(
+                  half2_t, __builtin_amdgcn_cvt_pkrtz(r0 - (float)mid[0], r1 - (float)mid[1]));
+#pragma unroll
+              for (int e = 0; e < 2; ++e)
+                pa[4 * u + i + e] = hi[e], pm[4 * u + i + e] = mid[e], pl[4 * u + i + e] = low[e];
+            }
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) {
+            const half8_t vb = v_frag(T, dt);
+            rest[dt] = mfma16x16x32(vb, pl, rest[dt]);
+            rest[dt] = mfma16x16x32(vb, pm, rest[dt]);
+            o[dt] = mfma16x16x32(vb, pa, o[dt]);
+          }
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            vb[i] = h0[i];
-            vb[4 + i] = h1[i];
+            o[dt][i] = fmaf(rest[dt][i], 1.f / 1024.f, o[dt][i]);
+            sum += o[dt][i];
           }
-          o[dt] = mfma16x16x32(vb, pa, o[dt]);
-          o[dt] = mfma16x16x32(vb, pl, o[dt]);
+        // An infinite V times a part that is 0 is NaN where the whole weight
+        // gives an infinity: the block again, in fp32 products (v_mfma_f32_
+        // 16x16x4_f32, k = g: key 16 T + 4 g + i).  They take 25% to 30% of the
+        // kernel's time, so they are kept for this case.
+        if (__builtin_amdgcn_ballot_w64(sum != sum) != 0) {  // uniform
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) o[dt] = before[dt];
+#pragma unroll
+          for (int T = 0; T < KB; ++T)
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+              const half4_t vt = v_tile(T, dt);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) o[dt] = mfma16x16x4f32((float)vt[i], acc[T][i], o[dt]);
+            }
         }
       }
     }
   }
   if (qg < L) {
-    const float inv = 1.0f / rows_sum(l_run);
+    const float inv = 1.0f / (kScaleP * rows_sum(l_run));
     half_t* orow = out + (((int64_t)b * L + qg) * H + h) * 64;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
@@ -955,7 +1031,12 @@ int launch_fused_attention_general(const void* q, const void* k, const void* v, 
   if (B * H * L == 0) return GD_OK;
   if (general_mfma_ok(D, L, P, error_flag, {q, k, v, pos_key, pos_query, c2p, p2c, key_mask, out})) {
     const dim3 grid((unsigned)(B * H * ((L + 63) / 64)));
-    const auto kernel = L % 4 == 0 ? fused_attention_mfma_kernel<true> : fused_attention_mfma_kernel<false>;
+    // Lengths that are a multiple of 16 take the weights in two parts (4% to 9%
+    // faster), as they always have; the others kept fp32 weights on the
+    // per-query kernels, so they keep all bits here.
+    const auto kernel = L % 16 == 0  ? fused_attention_mfma_kernel<true, false>
+                        : L % 4 == 0 ? fused_attention_mfma_kernel<true, true>
+                                     : fused_attention_mfma_kernel<false, true>;
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, static_cast<const half_t*>(q),
                        static_cast<const half_t*>(k), static_cast<const half_t*>(v),
                        static_cast<const half_t*>(pos_key), static_cast<const half_t*>(pos_query), c2p, p2c,

@@ -780,6 +780,55 @@ def test_fused_attention_all_masked_row_is_the_mean_of_v(L):
     assert np.all(np.abs(got - want) <= bound), (np.abs(got - want) - bound).max()
 
 
+def _one_high_key(L, H=2, gap=18.0):
+    """q, k, scale, tables and indices of rows whose key 0 scores exactly `gap` above all others, which score 0."""
+    q = np.zeros((1, H, L, 64), np.float16)
+    k = np.zeros((1, H, L, 64), np.float16)
+    q[..., 0] = 4.0
+    k[:, :, 0, 0] = gap
+    pkh, pqh = (np.zeros((H, 512, 64), np.float16) for _ in range(2))
+    idx = np.zeros((H, L, L), np.int32)
+    return q, k, pkh, pqh, idx, idx, np.zeros((1, L), np.float16), 0.25
+
+
+@pytest.mark.parametrize("L", [3, 63, 70, 200, 333, 511])
+def test_fused_attention_small_weights_keep_their_bits(L):
+    """At lengths that are no multiple of 16 a probability is held in fp32:
+    e^-18 (2^-26) beside a key of weight 1 whose V is 0 still contributes.
+    Bound: half an fp16 ulp and the fp32 rounding of weights and sums, (L +
+    64) of 2^-24 of the sum of |w v| (an exponent of up to 26, L terms)."""
+    q, k, pkh, pqh, c2p, p2c, key_mask, scale = _one_high_key(L)
+    H = q.shape[1]
+    v = (np.random.default_rng(L).uniform(0.5, 1.0, (1, H, L, 64)) * 65504).astype(np.float16)
+    v[:, :, 0] = 0
+    v[:, :, 1::2, 32:] *= -1
+    args = (q, k, v, pkh, pqh, c2p, p2c, key_mask)
+    want = O.fused_attention_kernel(*args, scale, round16=False)
+    mag = O.fused_attention_kernel(q, k, np.abs(v), *args[3:], scale, round16=False)
+    got = host(fk().fused_attention(*map(dev, args), scale, 1, H, L, 64, 512))
+    assert np.abs(want).max() > 5e-4
+    bound = 0.5 * ulp16(want) + (L + 64) * 2.0 ** -24 * mag
+    assert np.all(np.abs(got - want) <= bound), (np.abs(got - want) / bound).max()
+
+
+@pytest.mark.parametrize("L", [3, 63, 70, 200, 333, 511])
+def test_fused_attention_infinite_values(L):
+    """An infinite V of a key with a positive weight is an infinite output
+    (of its sign, in its column and no other), whatever bits the weight has;
+    two of opposite sign are NaN, as in the fp32 sum."""
+    q, k, pkh, pqh, c2p, p2c, key_mask, scale = _one_high_key(L)
+    H = q.shape[1]
+    v = np.random.default_rng(L).standard_normal((1, H, L, 64)).astype(np.float16)
+    v[0, 0, 0, 5] = np.inf        # weight 1
+    v[0, 0, L - 1, 6] = -np.inf   # weight e^-18
+    v[0, 0, 0, 7], v[0, 0, 1, 7] = np.inf, -np.inf
+    got = host(fk().fused_attention(*map(dev, (q, k, v, pkh, pqh, c2p, p2c, key_mask)), scale, 1, H, L, 64, 512))
+    assert np.all(got[0, :, 0, 5] == np.inf) and np.all(got[0, :, 0, 6] == -np.inf)
+    assert np.all(np.isnan(got[0, :, 0, 7]))
+    got[0, :, 0, 5:8] = 0
+    assert np.all(np.isfinite(got))
+
+
 def test_general_index_kernels_clamp_out_of_range_indices():
     """Indices outside [0, P) read the nearest table row (the per-query
     kernels' rule, kept by the matrix-core kernels)."""
