@@ -975,10 +975,13 @@ __global__ void relative_index_table_kernel(int32_t* __restrict__ out, int n, in
 // The matrix-core kernels read q, k, v and the table rows in 16-byte pieces
 // and, where L allows, the c2p indices and the key mask four at a time, and
 // store pieces of up to 16 bytes of the output; both entry points hold every
-// operand to 16-byte alignment, as the header states.
-bool general_mfma_ok(int64_t D, int64_t L, int64_t P, const int32_t* error_flag,
+// operand to 16-byte alignment, as the header states.  A launch holds fewer
+// than 2^32 threads: up to three queries in a workgroup of 256 threads reach
+// that before the per-query kernels' 64 threads a query do, so `groups` of them
+// (at most) that do not fit leave the call to those.
+bool general_mfma_ok(int64_t D, int64_t L, int64_t P, int64_t groups, const int32_t* error_flag,
                      std::initializer_list<const void*> ptrs) {
-  if (D != 64 || L > 512 || P > 65536 || error_flag != nullptr) return false;
+  if (D != 64 || L > 512 || P > 65536 || groups >= (int64_t{1} << 32) / 256 || error_flag != nullptr) return false;
   for (const void* p : ptrs)
     if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
   return true;
@@ -991,15 +994,17 @@ int launch_relative_bias_general(const void* q, const void* k, const void* pos_k
                                  int64_t H, int64_t L, int64_t D, int64_t P, void* out, int32_t* error_flag,
                                  hipStream_t stream) {
   if (B * H * L == 0) return GD_OK;
-  if (general_mfma_ok(D, L, P, error_flag, {q, k, pos_key, pos_query, c2p, p2c, key_mask, out})) {
-    // Batch rows per workgroup: the fewest that leave one round of the two
-    // workgroups a CU holds (a single one takes the form of three per CU).  A workgroup's indices and table rows cost it about
-    // 7 us and each batch row 2 us (B = 32, L = 256, 8,192 tiles: 1, 2, 4, 8, 16
-    // and 32 rows per workgroup take 133, 81, 55, 43, 36 and 45 us).
-    const int64_t blocks = (L + 63) / 64, tiles = H * blocks * blocks, slots = 2 * kGenCus;
-    const int64_t want = std::min(B, (B * tiles + slots - 1) / slots);
-    const int64_t nb = (B + (B + want - 1) / want - 1) / ((B + want - 1) / want);  // in even groups
-    const dim3 grid((unsigned)(tiles * ((B + nb - 1) / nb)));
+  // Batch rows per workgroup: the fewest that leave one round of the two
+  // workgroups a CU holds (all of them at most; a single one takes the form of
+  // three per CU).  A workgroup's indices and table rows cost it about 7 us and
+  // each batch row 2 us (B = 32, L = 256, 8,192 tiles: 1, 2, 4, 8, 16 and 32
+  // rows per workgroup take 133, 81, 55, 43, 36 and 45 us).
+  const int64_t blocks = (L + 63) / 64, tiles = H * blocks * blocks, slots = 2 * kGenCus;
+  const int64_t want = std::min(B, (B * tiles + slots - 1) / slots);
+  const int64_t nb = (B + (B + want - 1) / want - 1) / ((B + want - 1) / want);  // in even groups
+  const int64_t groups = tiles * ((B + nb - 1) / nb);
+  if (general_mfma_ok(D, L, P, groups, error_flag, {q, k, pos_key, pos_query, c2p, p2c, key_mask, out})) {
+    const dim3 grid((unsigned)groups);
     auto pick = [&](auto multi) {
       constexpr bool M = decltype(multi)::value;
       return L % 8 == 0   ? relative_bias_mfma_kernel<8, M>
@@ -1029,8 +1034,9 @@ int launch_fused_attention_general(const void* q, const void* k, const void* v, 
                                    float scale, int64_t B, int64_t H, int64_t L, int64_t D, int64_t P, void* out,
                                    int32_t* error_flag, hipStream_t stream) {
   if (B * H * L == 0) return GD_OK;
-  if (general_mfma_ok(D, L, P, error_flag, {q, k, v, pos_key, pos_query, c2p, p2c, key_mask, out})) {
-    const dim3 grid((unsigned)(B * H * ((L + 63) / 64)));
+  const int64_t groups = B * H * ((L + 63) / 64);
+  if (general_mfma_ok(D, L, P, groups, error_flag, {q, k, v, pos_key, pos_query, c2p, p2c, key_mask, out})) {
+    const dim3 grid((unsigned)groups);
     // Lengths that are a multiple of 16 take the weights in two parts (4% to 9%
     // faster), as they always have; the others kept fp32 weights on the
     // per-query kernels, so they keep all bits here.

@@ -829,6 +829,30 @@ def test_fused_attention_infinite_values(L):
     assert np.all(np.isfinite(got))
 
 
+@pytest.mark.parametrize("B,H", [(2 ** 20, 16), (1, 2 ** 24)])
+def test_general_index_kernels_many_short_rows(B, H):
+    """2^24 rows of one query: more workgroups of 256 threads than a launch
+    may hold, which the per-query kernels' workgroups of 64 still fit.  One
+    key: the attention is V itself, the bias one sum."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(H)
+    q, k = (torch.randn((B, H, 1, 64), generator=g, device="cuda", dtype=torch.float16) for _ in range(2))
+    pk, pq = (torch.randn((H, 1, 64), generator=g, device="cuda", dtype=torch.float16) for _ in range(2))
+    idx = torch.zeros((H, 1, 1), dtype=torch.int32, device="cuda")
+    mask = torch.zeros((B, 1), dtype=torch.float16, device="cuda")
+    args = (pk, pq, idx, idx, mask, 0.25, B, H, 1, 64, 1)
+    assert torch.equal(fk().fused_attention(q, k, q, *args).view(B, H, 64), q.view(B, H, 64))
+    bias = fk().relative_bias(q, k, *args).view(B, H)
+    b, h = (torch.randint(0, n, (4096,), generator=g, device="cuda") for n in (B, H))
+    b[:2], h[:2] = torch.tensor([0, B - 1]), torch.tensor([0, H - 1])
+    qd, kd, pkd, pqd = (t.double() for t in (q[b, h, 0], k[b, h, 0], pk[h, 0], pq[h, 0]))
+    want = (qd * pkd + kd * pqd).sum(-1) * 0.25
+    # one fp16 rounding of an fp32 sum of 128 products
+    bound = 0.5 * torch.from_numpy(ulp16(want.cpu().numpy())).cuda() + \
+        0.25 * 128 * 2.0 ** -24 * ((qd * pkd).abs() + (kd * pqd).abs()).sum(-1)
+    assert torch.all((bias[b, h].double() - want).abs() <= bound)
+
+
 def test_general_index_kernels_clamp_out_of_range_indices():
     """Indices outside [0, P) read the nearest table row (the per-query
     kernels' rule, kept by the matrix-core kernels)."""
