@@ -129,18 +129,27 @@ __global__ __launch_bounds__(64) void fused_attention_general_kernel(
 // through LDS tables of 80 columns, and each score takes one term from each at
 // its index.  C2P rows are read by the wave that writes them; P2C rows by all
 // four, so they alternate between two tables with one barrier per batch row.
-// Wider spans (arbitrary index tensors) run further windows over the same
-// tables, a position outside the window at hand reading a -0 column.  A score
-// is (-0 + c2p) + p2c, term by term the reference's fp32 sum.  Indices outside
-// [0, P) are clamped, as the per-query kernel does.  Queries and keys past L
-// repeat the last one (indices of a valid pair of the tile); their scores are
-// not stored.
+// Wider spans (arbitrary index tensors) run windows of 128 or 192 table rows, a
+// position outside the window at hand reading a -0 column.  A score is (-0 +
+// c2p) + p2c, term by term the reference's fp32 sum.  Indices outside [0, P)
+// are clamped, as the per-query kernel does.  Queries and keys past L repeat
+// the last one (indices of a valid pair of the tile); their scores are not
+// stored.
 //
-// Bound by the batch row's chain (MFMA, table, gather, barrier, store) with
-// two waves per SIMD (230-247 VGPRs).  B = 32, H = 16, L = 256: 36.4 us
-// against 72.5 us of a kernel that read indices and table rows for every batch
-// row and ran 64-row windows of either table, a gather per window; at 5 TB/s
-// its 111 MB take 22 us.
+// A workgroup of one batch row uses a table row once, so it takes the rows
+// through LDS in whole lines, one window of 128 for all four waves: a fragment
+// load from global memory touches 16 half lines for every 16 lanes (64 address
+// lookups a wave), which bound that form at 3.3 us per workgroup and CU (B = 1,
+// H = 16, L = 512: 18.1 us so, 14.5 through LDS; L = 256: 6.4 and 6.0).
+//
+// Several batch rows are bound by the batch row's chain (MFMA, table, gather,
+// barrier, store) with two waves per SIMD (250 VGPRs).  B = 32, H = 16, L =
+// 256: 36 us against 71 us of a kernel that read indices and table rows for
+// every batch row and ran 64-row windows of either table, a gather per window;
+// at 5 TB/s its 111 MB take 22 us.  Random indices (the whole table for every
+// tile): B = 1, L = 64 to 512 13.0 to 32.5 us, B = 32, L = 256 199 us (that
+// kernel 18.6 to 33.7 and 184; each wave reading its own windows of 80 rows
+// from global memory 27 to 88 and 540).
 // ---------------------------------------------------------------------------
 constexpr int64_t kGenCus = 256;  // compute units of the device the grids are sized for
 constexpr int kGenKeyBlocks = 4;  // 16-key blocks per key block (64 keys)
@@ -149,6 +158,11 @@ constexpr int kBiasCols = 16 * kBiasTiles;
 // fp32 row stride of the tables: float4 stores of 8 consecutive rows hit 32
 // distinct banks; column kBiasCols holds the -0 of a position outside the window.
 constexpr int kBiasStride = kBiasCols + 4;
+
+constexpr int kGenWin = 128;  // table rows per window in LDS
+
+// 64-half rows in LDS: 16-byte chunk `chunk` of row `row`.
+__device__ __forceinline__ int gen_swz(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
 // Least of a wave's values (VALU moves, no LDS round trips).
 template <int CTRL>
@@ -162,9 +176,8 @@ __device__ __forceinline__ int gen_wave_min(int v) {
              min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
-// Workgroups per CU of the form for one batch row (four would spill: B = 1, L =
-// 512 takes 18.3 us with three, 24.4 us with four).
-constexpr int kBiasOneWaves = 3;
+// Workgroups per CU (waves per SIMD) the registers and LDS are held to.
+constexpr int bias_waves(bool multi) { return multi ? 2 : 3; }
 
 // W: the largest of 8, 4, 2 and 1 that divides L, the halfs of the output
 // pieces (every row starts aligned to one); from 4 on the c2p indices and the
@@ -172,15 +185,24 @@ constexpr int kBiasOneWaves = 3;
 // walks several batch rows.  With one there is nothing to keep: P2C takes the
 // C2P rows' place, and kBiasOneWaves workgroups share a CU.
 template <int W, bool MULTI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 : kBiasOneWaves, MULTI ? 2 : kBiasOneWaves))) void relative_bias_mfma_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bias_waves(MULTI), bias_waves(MULTI)))) void relative_bias_mfma_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ pos_key,
     const half_t* __restrict__ pos_query, const int32_t* __restrict__ c2p_idx, const int32_t* __restrict__ p2c_idx,
     const half_t* __restrict__ key_mask, float scale, int B, int H, int L, int P, int nb, half_t* __restrict__ out) {
   constexpr int KB = kGenKeyBlocks;
   constexpr bool VEC = W >= 4;
-  __shared__ __attribute__((aligned(16))) float ctab[64 * kBiasStride];     // C2P [query][column]
-  __shared__ __attribute__((aligned(16))) float ptabs[MULTI ? 2 : 1][MULTI ? 64 * kBiasStride : 4];  // P2C [key][column]
-  auto ptab = [&](int i) -> float* { return MULTI ? ptabs[i] : ctab; };
+  // C2P [query][column] and P2C [key][column]: MULTI keeps two tables of the
+  // latter, in an array of their own (so that their stores and C2P's reads may
+  // pass each other); with one batch row P2C takes C2P's place, and a window
+  // of posK rows and one of posQ rows follow.  Wide spans: a window of kWin
+  // rows, and one table of kWin columns.
+  constexpr int kTab = 64 * kBiasStride, kRows = kGenWin * 64 / 2;  // floats
+  constexpr int kWin = MULTI ? 192 : kGenWin, kWideStride = kWin + 4;
+  constexpr int kWideRows = kWin * 64 / 2, kWideTab = 64 * kWideStride;
+  constexpr int kOneRow = kTab + 2 * kRows > kWideRows + kWideTab ? kTab + 2 * kRows : kWideRows + kWideTab;
+  __shared__ __attribute__((aligned(1024))) float ctab[!MULTI ? kOneRow : kTab > kWideRows ? kTab : kWideRows];
+  __shared__ __attribute__((aligned(16))) float ptabs[!MULTI ? 4 : 2 * kTab > kWideTab ? 2 * kTab : kWideTab];
+  auto ptab = [&](int i) -> float* { return MULTI ? ptabs + i * kTab : ctab; };
   __shared__ int ranges[4][2 + 2 * KB];  // per wave: least c2p, -c2p, then p2c and -p2c of each 16-key block
   // Workgroup -> (h, 64-query block qb, key block ky, batch rows b0 ..).
   // Workgroups go to the 8 XCDs round-robin; with H a multiple of 8, XCD x
@@ -211,9 +233,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
   const int qr = qw + lc < L ? qw + lc : L - 1;  // this lane's query (keys 4 g .. 4 g + 3 of a block)
   const int kw = 64 * ky + 16 * wave + lc;       // this lane's key of the wave's P2C rows
   const int kr = kw < L ? kw : L - 1;
-  // A wave with neither a query nor a P2C key ends here: the barriers below
-  // wait for the waves that go on, and nothing reads this one's rows.
-  if (qw >= L && 64 * ky + 16 * wave >= L) return;
   const half_t* pkh = pos_key + (int64_t)h * P * 64;
   const half_t* pqh = pos_query + (int64_t)h * P * 64;
   const int32_t* c2ph = c2p_idx + (int64_t)h * L * L;
@@ -230,21 +249,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
     half8_t q[2], k[2];
     half4_t mask[KB];
   };
-  auto fetch = [&](int b, Row& x) {
-    const int64_t bh = (int64_t)b * H + h;
-    row_frags(q + bh * L * 64, qr, x.q);
-    row_frags(k + bh * L * 64, kr, x.k);
+  auto fetch_mask = [&](int b, half4_t (&mask)[KB]) {
     const half_t* mrow = key_mask + (int64_t)b * L;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const int key = key_of(kb);
       if constexpr (VEC) {
-        x.mask[kb] = *reinterpret_cast<const half4_t*>(mrow + (uint32_t)(key < L ? key : L - 4));
+        mask[kb] = *reinterpret_cast<const half4_t*>(mrow + (uint32_t)(key < L ? key : L - 4));
       } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x.mask[kb][j] = mrow[(uint32_t)(key + j < L ? key + j : L - 1)];
+        for (int j = 0; j < 4; ++j) mask[kb][j] = mrow[(uint32_t)(key + j < L ? key + j : L - 1)];
       }
     }
+  };
+  auto fetch = [&](int b, Row& x) {
+    const int64_t bh = (int64_t)b * H + h;
+    row_frags(q + bh * L * 64, qr, x.q);
+    row_frags(k + bh * L * 64, kr, x.k);
+    fetch_mask(b, x.mask);
   };
 
   // ---- once: indices, their ranges, table rows ----
@@ -272,12 +294,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
   auto tile_frags = [&](const half_t* table, int row0, half8_t (&f)[2]) {
     row_frags(table, row0 + lc < P ? row0 + lc : P - 1, f);
   };
-  half8_t ct[kBiasTiles][2], pt[kBiasTiles][2];
+  // A window of table rows from row `base` on, in whole lines through
+  // registers into LDS, and the 16-row tile there from its row r0 on.
+  auto fetch_window = [&](const half_t* table, int base, half8_t (&x)[kWin / 32]) {
+#pragma unroll
+    for (int i = 0; i < kWin / 32; ++i) {
+      const int row = base + 32 * i + (int)(threadIdx.x >> 3);
+      x[i] = *reinterpret_cast<const half8_t*>(table + (uint32_t)((row < P ? row : P - 1) * 64 + 8 * (threadIdx.x & 7)));
+    }
+  };
+  auto put_window = [&](const half8_t (&x)[kWin / 32], float* rows) {
+#pragma unroll
+    for (int i = 0; i < kWin / 32; ++i)
+      *reinterpret_cast<half8_t*>(reinterpret_cast<half_t*>(rows) + gen_swz(32 * i + (int)(threadIdx.x >> 3), threadIdx.x & 7)) =
+          x[i];
+  };
+  auto window_frags = [&](const float* rows, int r0, half8_t (&f)[2]) {
+    f[0] = *reinterpret_cast<const half8_t*>(reinterpret_cast<const half_t*>(rows) + gen_swz(r0 + lc, g));
+    f[1] = *reinterpret_cast<const half8_t*>(reinterpret_cast<const half_t*>(rows) + gen_swz(r0 + lc, 4 + g));
+  };
+  half8_t ct[kBiasTiles][2], pt[kBiasTiles][2];  // MULTI only
   uint32_t cp[KB][4];  // the clamped indices, c2p | p2c << 16
   auto c_of = [](uint32_t x) { return (int)(x & 0xFFFFu); };
   auto p_of = [](uint32_t x) { return (int)(x >> 16); };
   Row cur, nxt;
-  fetch(b0, nxt);
+  if constexpr (MULTI && VEC) fetch(b0, nxt);  // (the others would spill)
   {
     int c_mn = P, c_mx = 0, p_mn[KB], p_mx[KB];
 #pragma unroll
@@ -295,7 +336,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
     r[0] = gen_wave_min(c_mn), r[1] = gen_wave_min(-c_mx);
     // the c2p rows need no other wave's range: in flight from here
 #pragma unroll
-    for (int tp = 0; tp < kBiasTiles; ++tp) tile_frags(pkh, r[0] + 16 * tp, ct[tp]);
+    for (int tp = 0; MULTI && tp < kBiasTiles; ++tp) tile_frags(pkh, r[0] + 16 * tp, ct[tp]);
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) r[2 + 2 * kb] = gen_wave_min(p_mn[kb]), r[3 + 2 * kb] = gen_wave_min(-p_mx[kb]);
     if (lane == 0) {
@@ -304,29 +345,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
     }
   }
   stage_barrier();
-  // least index of the wave's c2p and of each block's p2c, greatest spans
-  int c_lo = 0;
-  int p_lo[KB], c_end = 0, p_all = P, p_end = 0;
+  // least index of the wave's c2p, of every wave's and of each block's p2c,
+  // and the greatest
+  int c_lo = 0, c_all = P, c_end = 0;
+  int p_lo[KB], p_all = P, p_end = 0;
   bool narrow = true;  // uniform over the workgroup: every window is one
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
-    if (64 * qb + 16 * w >= L && w != wave) continue;  // no query: its indices are another wave's
     const int lo = __builtin_amdgcn_readfirstlane(ranges[w][0]), hi = -__builtin_amdgcn_readfirstlane(ranges[w][1]);
     narrow = narrow && hi - lo < kBiasCols;
-    if (w == wave) c_lo = lo, c_end = hi;
+    if (w == wave) c_lo = lo;
+    c_all = min(c_all, lo), c_end = max(c_end, hi);
   }
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     int lo = P, hi = P;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      if (64 * qb + 16 * w >= L) continue;
-      lo = min(lo, ranges[w][2 + 2 * kb]), hi = min(hi, ranges[w][3 + 2 * kb]);
-    }
+    for (int w = 0; w < 4; ++w) lo = min(lo, ranges[w][2 + 2 * kb]), hi = min(hi, ranges[w][3 + 2 * kb]);
     p_lo[kb] = __builtin_amdgcn_readfirstlane(lo);
     hi = -__builtin_amdgcn_readfirstlane(hi);
     narrow = narrow && hi - p_lo[kb] < kBiasCols;
     p_all = min(p_all, p_lo[kb]), p_end = max(p_end, hi);
+  }
+  if constexpr (!MULTI) {
+    narrow = narrow && c_end - c_all < kGenWin && p_end - p_all < kGenWin;
+    // (a wave's tiles stay inside the workgroup's window)
+    c_lo = min(c_lo, c_all + kGenWin - kBiasCols);
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) p_lo[kb] = min(p_lo[kb], p_all + kGenWin - kBiasCols);
   }
   // One tile's products into a table row's columns.
   auto product = [&](const half8_t (&a)[2], const half8_t (&f)[2], float* row, int tp) {
@@ -338,10 +384,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
   float* const crow = ctab + (16 * wave + lc) * kBiasStride;
   const int b_end = !MULTI ? b0 + 1 : (b0 + nb < B ? b0 + nb : B);
 
+  auto await_next = [&] {
+    asm volatile("" : "+v"(nxt.q[0]), "+v"(nxt.q[1]), "+v"(nxt.k[0]), "+v"(nxt.k[1]));
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(nxt.mask[kb]));
+  };
+
   // ---- scores: (c2p + p2c) * scale, masked keys -65504, staged through the
-  // wave's C2P rows into row pieces of up to 128 bytes ----
-  auto finish = [&](int b, const float (&acc)[KB][4], const half4_t (&mask)[KB]) {
-    half_t* const stage = reinterpret_cast<half_t*>(ctab + 16 * wave * kBiasStride);
+  // wave's table rows into row pieces of up to 128 bytes ----
+  auto finish = [&](auto prefetched, int b, const float (&acc)[KB][4], const half4_t (&mask)[KB], float* own) {
+    half_t* const stage = reinterpret_cast<half_t*>(own);
     wave_lds_sync();
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
@@ -359,11 +411,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
     half_t* const orow = out + (((int64_t)b * H + h) * L + qw) * L;  // uniform
     // (the next batch row's loads are waited for here: behind the stores, the
     // wait would be for the stores too)
-    if constexpr (MULTI) {
-      asm volatile("" : "+v"(nxt.q[0]), "+v"(nxt.q[1]), "+v"(nxt.k[0]), "+v"(nxt.k[1]));
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(nxt.mask[kb]));
-    }
+    if constexpr (decltype(prefetched)::value) await_next();
 #pragma unroll
     for (int r0 = 0; r0 < 16; r0 += ROWS)
       if (qw + r0 + r < L && 64 * ky + cc < L)
@@ -376,25 +424,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
     int p_own = p_lo[0];
 #pragma unroll
     for (int kb = 1; kb < KB; ++kb) p_own = wave == kb ? p_lo[kb] : p_own;
+    if constexpr (!(MULTI && VEC)) fetch(b0, nxt);
+    if constexpr (MULTI) {
 #pragma unroll
-    for (int tp = 0; tp < kBiasTiles; ++tp) tile_frags(pqh, p_own + 16 * tp, pt[tp]);
-    // (used here, so that they are waited for here: a wait inside the loop
-    // would also wait for the next batch row's loads, issued after them)
+      for (int tp = 0; tp < kBiasTiles; ++tp) tile_frags(pqh, p_own + 16 * tp, pt[tp]);
+      // (used here, so that they are waited for here: a wait inside the loop
+      // would also wait for the next batch row's loads, issued after them)
 #pragma unroll
-    for (int tp = 0; MULTI && tp < kBiasTiles; ++tp)
-      asm volatile("" : "+v"(ct[tp][0]), "+v"(ct[tp][1]), "+v"(pt[tp][0]), "+v"(pt[tp][1]));
+      for (int tp = 0; tp < kBiasTiles; ++tp)
+        asm volatile("" : "+v"(ct[tp][0]), "+v"(ct[tp][1]), "+v"(pt[tp][0]), "+v"(pt[tp][1]));
+      await_next();
+    } else {
+      half8_t x[kWin / 32], y[kWin / 32];
+      fetch_window(pkh, c_all, x), fetch_window(pqh, p_all, y);
+      put_window(x, ctab + kTab), put_window(y, ctab + kTab + kRows);
+      stage_barrier();
+    }
     int pbuf = 0;
     for (int b = b0; b < b_end; ++b) {  // uniform
       cur = nxt;
       if (b + 1 < b_end) fetch(b + 1, nxt);
       float* const pt_b = ptab(pbuf);
       float* const prow = pt_b + (16 * wave + lc) * kBiasStride;
+      // one table's tiles against the wave's rows: from registers, or from row r0 of a window on
+      auto products = [&](const half8_t (&f)[kBiasTiles][2], const float* rows, int r0, const half8_t (&a)[2], float* row) {
 #pragma unroll
-      for (int tp = 0; tp < kBiasTiles; ++tp) product(ct[tp], cur.q, crow, tp);
-      if constexpr (MULTI) {
-#pragma unroll
-        for (int tp = 0; tp < kBiasTiles; ++tp) product(pt[tp], cur.k, prow, tp);
-      }
+        for (int tp = 0; tp < kBiasTiles; ++tp) {
+          if constexpr (MULTI) {
+            product(f[tp], a, row, tp);
+          } else {
+            half8_t x[2];
+            window_frags(rows, r0 + 16 * tp, x);
+            product(x, a, row, tp);
+          }
+        }
+      };
+      products(ct, ctab + kTab, c_lo - c_all, cur.q, crow);
+      if constexpr (MULTI) products(pt, nullptr, 0, cur.k, prow);
       wave_lds_sync();
       float acc[KB][4];
 #pragma unroll
@@ -403,8 +469,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
         for (int j = 0; j < 4; ++j) acc[kb][j] = crow[c_of(cp[kb][j]) - c_lo];
       if constexpr (!MULTI) {
         wave_lds_sync();
-#pragma unroll
-        for (int tp = 0; tp < kBiasTiles; ++tp) product(pt[tp], cur.k, prow, tp);
+        products(pt, ctab + kTab + kRows, p_own - p_all, cur.k, prow);
       }
       stage_barrier();  // P2C rows visible; the last batch row's P2C reads are a barrier back
 #pragma unroll
@@ -413,57 +478,75 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
         for (int j = 0; j < 4; ++j)
           acc[kb][j] += pt_b[(16 * kb + 4 * g + j) * kBiasStride + (p_of(cp[kb][j]) - p_lo[kb])];
       if constexpr (!MULTI) stage_barrier();  // the scores are staged in the rows that were read
-      finish(b, acc, cur.mask);
+      finish(std::bool_constant<MULTI>{}, b, acc, cur.mask, ctab + 16 * wave * kBiasStride);
       pbuf ^= 1;
     }
   } else {
+    // Wide spans: windows of kWin rows of either table in turn, a position
+    // outside the window at hand reading a -0 column.  Wave w takes the
+    // window's tiles w, w + 4, .. against all 64 queries or keys, so that a
+    // table row is read once for the workgroup, and the next window comes during
+    // the products and the gather.
+    float* const wtab = MULTI ? ptabs : ctab + kWideRows;
+    half8_t x[kWin / 32];
+    auto windows = [&](const half_t* table, int lo, int end, const half_t* base, int row0, auto&& gather) {
+      // (opaque: with both tables' fragments and addresses hoisted out of the
+      // loops, registers would spill)
+      int row = row0 + lc;
+      asm volatile("" : "+v"(row));
+      half8_t r64[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) row_frags(base, row + 16 * u < L ? row + 16 * u : L - 1, r64[u]);
+      fetch_window(table, lo, x);
+      if (MULTI) put_window(x, ctab);
+      for (int w0 = lo; w0 <= end; w0 += kWin) {  // uniform
+        if (!MULTI) put_window(x, ctab);
+        stage_barrier();  // (and every wave is past the last window's gather)
+        if (w0 + kWin <= end) fetch_window(table, w0 + kWin, x);
+#pragma unroll
+        for (int tp = 0; tp < kWin / 16; tp += 4) {
+          if (w0 + 16 * (wave + tp) > end) continue;  // uniform
+          half8_t f[2];
+          window_frags(ctab, 16 * (wave + tp), f);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) product(f, r64[u], wtab + (16 * u + lc) * kWideStride, wave + tp);
+        }
+        stage_barrier();
+        // (before the gather where two workgroups share a CU: 199 against 207 us;
+        // with three after it: 32 against 34 us)
+        if (MULTI && w0 + kWin <= end) put_window(x, ctab);
+        gather(w0);
+      }
+    };
+    float* const own = wtab + (16 * wave + lc) * kWideStride;
     for (int b = b0; b < b_end; ++b) {  // uniform
-      cur = nxt;
-      if (b + 1 < b_end) fetch(b + 1, nxt);
-      // (the windows' addresses stay inside the loop: hoisting them all would
-      // spill registers)
-      int base = 0;
-      asm volatile("" : "+v"(base));
-      base = __builtin_amdgcn_readfirstlane(base);
-      int lo = c_lo + base, plo = p_all + base;
+      int zero = 0;  // (opaque, as above)
+      asm volatile("" : "+v"(zero));
+      zero = __builtin_amdgcn_readfirstlane(zero);
+      const int64_t bh = (int64_t)b * H + h;
       float acc[KB][4];
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[kb][j] = -0.0f;
-      if (lane < 16) crow[kBiasCols] = -0.0f;
-      for (; lo <= c_end; lo += kBiasCols) {  // uniform within the wave
-#pragma unroll
-        for (int tp = 0; tp < kBiasTiles; ++tp) {
-          half8_t f[2];
-          tile_frags(pkh, lo + 16 * tp, f);
-          product(f, cur.q, crow, tp);
-        }
-        wave_lds_sync();
+      if (lane < 16) own[kWin] = -0.0f;
+      windows(pkh, c_all + zero, c_end, q + bh * L * 64, 64 * qb, [&](int w0) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[kb][j] += crow[min((uint32_t)(c_of(cp[kb][j]) - lo), (uint32_t)kBiasCols)];
-        wave_lds_sync();
-      }
-      float* const prow = ptab(0) + (16 * wave + lc) * kBiasStride;
-      if (lane < 16) prow[kBiasCols] = -0.0f;
-      for (; plo <= p_end; plo += kBiasCols) {  // uniform over the workgroup
-#pragma unroll
-        for (int tp = 0; tp < kBiasTiles; ++tp) {
-          half8_t f[2];
-          tile_frags(pqh, plo + 16 * tp, f);
-          product(f, cur.k, prow, tp);
-        }
-        stage_barrier();
+          for (int j = 0; j < 4; ++j) acc[kb][j] += own[min((uint32_t)(c_of(cp[kb][j]) - w0), (uint32_t)kWin)];
+      });
+      windows(pqh, p_all + zero, p_end, k + bh * L * 64, 64 * ky, [&](int w0) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            acc[kb][j] += ptab(0)[(16 * kb + 4 * g + j) * kBiasStride + min((uint32_t)(p_of(cp[kb][j]) - plo), (uint32_t)kBiasCols)];
-        stage_barrier();
-      }
-      finish(b, acc, cur.mask);
+            acc[kb][j] += wtab[(16 * kb + 4 * g + j) * kWideStride + min((uint32_t)(p_of(cp[kb][j]) - w0), (uint32_t)kWin)];
+      });
+      half4_t mask[KB];
+      fetch_mask(b, mask);
+      stage_barrier();  // the scores are staged in the rows that were read
+      finish(std::false_type{}, b, acc, mask, wtab + 16 * wave * kWideStride);
     }
   }
 }
@@ -497,16 +580,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 2 :
 // parts 25.5, P . V in fp32 products 33.6, the per-query kernel 495); B = 32,
 // L = 256: 90 us (64-row windows, a gather per window: 97 us).
 // ---------------------------------------------------------------------------
-constexpr int kGenWin = 128;  // table rows per window
-
 typedef __attribute__((address_space(3))) half_t gen_lds_half_t;
 typedef short gen_short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) gen_short4_t gen_lds_short4_t;
 
 // A row of zeros: the V rows of keys past L.
 __device__ __attribute__((aligned(16))) const half_t g_zero_row[64] = {};
-
-__device__ __forceinline__ int gen_swz(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
 
 // VEC: L is a multiple of 4, so the c2p indices and the mask of four
 // consecutive keys are one aligned load.  EXACT: P . V takes all 24 bits of
@@ -995,13 +1074,18 @@ int launch_relative_bias_general(const void* q, const void* k, const void* pos_k
                                  hipStream_t stream) {
   if (B * H * L == 0) return GD_OK;
   // Batch rows per workgroup: the fewest that leave one round of the two
-  // workgroups a CU holds (all of them at most; a single one takes the form of
-  // three per CU).  A workgroup's indices and table rows cost it about 7 us and
-  // each batch row 2 us (B = 32, L = 256, 8,192 tiles: 1, 2, 4, 8, 16 and 32
-  // rows per workgroup take 133, 81, 55, 43, 36 and 45 us).
+  // workgroups a CU holds, all of them at most (B = 32, L = 256, 8,192 tiles: 1,
+  // 2, 4, 8, 16 and 32 rows per workgroup take 133, 81, 55, 43, 36 and 45 us).
+  // A round takes about 7 us for a workgroup's indices and table rows and 2 us
+  // for each batch row; the form for one batch row takes about 3 us and 3 us
+  // for each workgroup of a CU (256, 576 and 1,024 of them 6.0, 10.9 and 14.5
+  // us), which is less where several rows would need a second round (B = 2, L =
+  // 384, 1,152 tiles: 15.5 against 19.0 us).
   const int64_t blocks = (L + 63) / 64, tiles = H * blocks * blocks, slots = 2 * kGenCus;
   const int64_t want = std::min(B, (B * tiles + slots - 1) / slots);
-  const int64_t nb = (B + (B + want - 1) / want - 1) / ((B + want - 1) / want);  // in even groups
+  int64_t nb = (B + (B + want - 1) / want - 1) / ((B + want - 1) / want);  // in even groups
+  const int64_t rounds = (tiles * ((B + nb - 1) / nb) + slots - 1) / slots;
+  if (3.0 + 3.0 * (double)(B * tiles) / kGenCus < (double)rounds * (7.0 + 2.0 * (double)nb)) nb = 1;
   const int64_t groups = tiles * ((B + nb - 1) / nb);
   if (general_mfma_ok(D, L, P, groups, error_flag, {q, k, pos_key, pos_query, c2p, p2c, key_mask, out})) {
     const dim3 grid((unsigned)groups);

@@ -753,6 +753,40 @@ def test_general_index_kernels_any_length(L, P, H, B, relative):
     assert np.max(np.abs(got - want)) <= 2e-3  # one fp16 rounding of values below 4
 
 
+@pytest.mark.parametrize("relative", [True, False])
+@pytest.mark.parametrize("L,H,B", [(256, 16, 5), (252, 16, 5), (254, 16, 5), (253, 16, 5), (512, 3, 3)])
+def test_relative_bias_several_batch_rows(L, H, B, relative):
+    """Workgroups that walk several batch rows (more than 512 tiles of 64 x 64
+    over the batch), the last group a shorter one, at lengths that are a
+    multiple of 8, of 4, of 2 and odd, with one table window per tile and with
+    several; every batch row has its own Q, K and mask.  L = 512, H = 3: more
+    tiles than one round, one batch row a workgroup."""
+    P = 512
+    r = np.random.default_rng(2300 + L)
+    q, k = (r.standard_normal((B, H, L, 64)).astype(np.float16) for _ in range(2))
+    pkh, pqh = (r.standard_normal((H, P, 64)).astype(np.float16) for _ in range(2))
+    if relative:
+        rel = np.arange(L)[:, None] - np.arange(L)[None, :]
+        idx = np.clip(O.relative_bucket(rel) + 256, 0, P - 1).astype(np.int32)
+        c2p = np.broadcast_to(idx, (H, L, L)).copy()
+        p2c = np.broadcast_to(idx.T, (H, L, L)).copy()
+    else:
+        c2p = r.integers(0, P, size=(H, L, L)).astype(np.int32)
+        p2c = r.integers(0, P, size=(H, L, L)).astype(np.int32)
+    key_mask = np.where(r.random((B, L)) < 0.1, -65504.0, 0.0).astype(np.float16)
+    scale = O.scale_f32(64)
+    got = host(fk().relative_bias(*(dev(a) for a in (q, k, pkh, pqh, c2p, p2c, key_mask)), scale, B, H, L, 64, P))
+    masked = np.broadcast_to(key_mask[:, None, None, :] < -60000, got.shape)
+    assert np.all(got[masked] == -65504.0)
+    want = O.relative_bias_kernel(q, k, pkh, pqh, c2p, p2c, key_mask, scale)
+    # an fp32 sum of 129 products (8 units of 2^-24 per MFMA step of the terms' magnitudes, as above), one rounding
+    acc = 4.0 * 8.0 * 2.0 ** -24 * O.relative_bias_kernel(np.abs(q), np.abs(k), np.abs(pkh), np.abs(pqh), c2p, p2c,
+                                                            np.zeros_like(key_mask), scale, round16=False)
+    err = np.abs(got - want)[~masked]
+    bound = (np.maximum(ulp16(got), ulp16(want)) + acc)[~masked]
+    assert np.all(err <= bound + 1e-12), (err - bound).max()
+
+
 @pytest.mark.parametrize("L", [65, 200, 256, 333, 500, 512])
 def test_fused_attention_all_masked_row_is_the_mean_of_v(L):
     """With every key masked each weight is exp(-65504 - -65504) / L: the
