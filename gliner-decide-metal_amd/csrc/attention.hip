@@ -559,9 +559,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bias_waves(
 // of the wave's 16 x 64 positions on, as in the bias kernel; here each key
 // block needs fresh table rows, so a window of 128 rows of each table (the 64 x
 // 64 tile's relative positions span at most 127) comes by DMA for all four
-// waves.  Wider spans run further windows.  Every c2p window precedes every p2c
-// window, so a score accumulates (q.k + c2p) + p2c, the reference's fp32 sum,
-// term by term.
+// waves.  Wider spans run windows of 128 rows and columns one after the other,
+// the rows in whole lines, the next ones in flight (random indices: B = 1, L =
+// 512 97 us, B = 32, L = 256 230 us; 80 columns at a time, each window waited
+// for, 153 and 347; 64-row windows in a kernel of four workgroups per CU, 176
+// and 249).  Every c2p window precedes every p2c window, so a score accumulates
+// (q.k + c2p) + p2c, the reference's fp32 sum, term by term.
 //
 // Scores (masked keys -65504, keys past L -inf) feed an online softmax per
 // query row (running max seeded at -65504, the reference's seed), and P . V
@@ -576,7 +579,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bias_waves(
 // The next key block's windows, K and V rows come by DMA during the softmax and
 // P . V, its indices a block earlier; two barriers per block.
 // Bound by the block's chain of LDS round trips with two waves per SIMD (79 KB
-// of LDS, 240 and 248 VGPRs).  B = 8, H = 16, L = 200 (EXACT): 27.5 us (two
+// of LDS, 254 VGPRs).  B = 8, H = 16, L = 200 (EXACT): 27.5 us (two
 // parts 25.5, P . V in fp32 products 33.6, the per-query kernel 495); B = 32,
 // L = 256: 90 us (64-row windows, a gather per window: 97 us).
 // ---------------------------------------------------------------------------
@@ -597,10 +600,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int32_t* __restrict__ p2c_idx, const half_t* __restrict__ key_mask, float scale, int H, int L, int P,
     half_t* __restrict__ out) {
   constexpr int KB = kGenKeyBlocks;
-  __shared__ __attribute__((aligned(1024))) half_t rk[kGenWin * 64];    // window of posK rows
-  __shared__ __attribute__((aligned(1024))) half_t rq[kGenWin * 64];    // window of posQ rows
-  __shared__ __attribute__((aligned(1024))) half_t krows[64 * 64];      // K rows of the key block
-  __shared__ __attribute__((aligned(1024))) half_t vrows[2][64 * 64];   // V rows of this and the next key block
+  // K rows of the key block and windows of posK and posQ rows, whose place the
+  // table of kGenWin columns takes with wide spans.
+  constexpr int kBlock = 64 * 64, kWideStride = kGenWin + 4;
+  __shared__ __attribute__((aligned(1024))) half_t krows[kBlock + 2 * kGenWin * 64];
+  half_t* const rk = krows + kBlock;
+  half_t* const rq = rk + kGenWin * 64;
+  __shared__ __attribute__((aligned(1024))) half_t vrows[2][kBlock];    // V rows of this and the next key block
+  static_assert(64 * kWideStride * 2 <= kBlock + 2 * kGenWin * 64 && kGenWin * 64 <= 2 * 64 * kBiasStride, "wide spans fit");
   __shared__ __attribute__((aligned(16))) float tab[64 * kBiasStride];  // C2P [query][col], then P2C [key][col]
   __shared__ int ranges[2][4][2 + 2 * KB];  // per wave: least c2p, -c2p, then p2c and -p2c of each 16-key block
   // Workgroup -> (b, h, query block qb), heads to XCDs as in the bias kernel.
@@ -737,29 +744,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int kb = 1; kb < KB; ++kb) x.p_own = wave == kb ? x.p_block[kb] : x.p_own;
     return x;
   };
-  // DMA of `ROWS` rows, row r from src(r): lane l of a 1 KiB block brings
-  // physical chunk l % 8 of row l / 8.
+  // DMA of `ROWS` rows, halfs c .. c + 7 of row r from src(r, c): lane l of a 1
+  // KiB block brings physical chunk l % 8 of row l / 8.
   auto issue_rows = [&](auto rows_c, half_t* dst, auto&& src) {
     constexpr int BLOCKS = decltype(rows_c)::value / 32;  // 1 KiB blocks per wave
 #pragma unroll
     for (int j = 0; j < BLOCKS; ++j) {
       const int blk = wave * BLOCKS + j;
       const int row = 8 * blk + (lane >> 3);
-      load_lds16(src(row) + (((lane & 7) ^ ((row >> 1) & 7)) << 3), dst + blk * 512);
+      load_lds16(src(row, ((lane & 7) ^ ((row >> 1) & 7)) << 3), dst + blk * 512);
     }
   };
+  // (one 32-bit offset from a uniform base wherever that can be: 64-bit
+  // addresses of every block, kept over the key blocks, would spill)
   auto issue_window = [&](const half_t* table, half_t* dst, int base) {  // rows past P repeat row P - 1
     issue_rows(std::integral_constant<int, kGenWin>{}, dst,
-               [&](int row) { return table + (uint32_t)((base + row < P ? base + row : P - 1) * 64); });
+               [&](int row, int c) { return table + (uint32_t)((base + row < P ? base + row : P - 1) * 64 + c); });
   };
   auto issue_block = [&](int kyb) {  // K rows (past L: the last one) and V rows (past L: zeros)
-    issue_rows(std::integral_constant<int, 64>{}, krows, [&](int row) {
+    issue_rows(std::integral_constant<int, 64>{}, krows, [&](int row, int c) {
       const int key = 64 * kyb + row;
-      return kbase + (uint32_t)((key < L ? key : L - 1) * 64);
+      return kbase + (uint32_t)((key < L ? key : L - 1) * 64 + c);
     });
-    issue_rows(std::integral_constant<int, 64>{}, vrows[kyb & 1], [&](int row) {
+    issue_rows(std::integral_constant<int, 64>{}, vrows[kyb & 1], [&](int row, int c) {
       const int key = 64 * kyb + row;
-      return key < L ? vbase + (uint32_t)(key * 64) : g_zero_row;
+      return key < L ? vbase + (uint32_t)(key * 64 + c) : g_zero_row + c;
     });
   };
   // kBiasTiles tiles of 16 window rows from row `r0` on against the 16 rows
@@ -843,36 +852,76 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       wave_lds_sync();
       products(rq, rg.p_own - rg.p_lo, kp0, kp1);
     } else {
-      // Tiles wider than one window or one wave's columns: 80 columns of
-      // each table in turn, a position outside them reading a -0 column
-      // (x + -0 = x for every fp32 x).
-      if (lane < 16) own[kBiasCols] = -0.0f;
-      for (int w0 = rg.c_lo; w0 <= rg.c_hi; w0 += kBiasCols) {  // uniform
-        issue_window(pkh, rk, w0);
-        wait_vmcnt<0>();
+      // Tiles wider than one window or one wave's columns: windows of kGenWin
+      // rows of each table in turn, through registers into the table's place
+      // `tab`, the next one in flight meanwhile; a position outside them reads a
+      // -0 column (x + -0 = x for every fp32 x).
+      // (opaque: addresses hoisted out of the loop over the key blocks would
+      // spill registers there)
+      int tw = t;
+      asm volatile("" : "+v"(tw));
+      const int lw = tw & 15, gw = (tw >> 4) & 3, rw = tw >> 3, cw = tw & 7;
+      float* const wtab = reinterpret_cast<float*>(krows);
+      float* const wown = wtab + (16 * wave + lw) * kWideStride;
+      half_t* const rows = reinterpret_cast<half_t*>(tab);
+      half8_t x[kGenWin / 32];
+      auto fetch = [&](const half_t* table, int base) {
+#pragma unroll
+        for (int i = 0; i < kGenWin / 32; ++i) {
+          const int row = base + 32 * i + rw;
+          x[i] = *reinterpret_cast<const half8_t*>(table + (uint32_t)((row < P ? row : P - 1) * 64 + 8 * cw));
+        }
+      };
+      auto put = [&] {
+#pragma unroll
+        for (int i = 0; i < kGenWin / 32; ++i) *reinterpret_cast<half8_t*>(rows + gen_swz(32 * i + rw, cw)) = x[i];
+      };
+      auto wide_products = [&](half8_t f0, half8_t f1) {
+#pragma unroll
+        for (int tp = 0; tp < kGenWin / 16; ++tp) {
+          const half8_t a0 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * tp + lw, gw));
+          const half8_t a1 = *reinterpret_cast<const half8_t*>(rows + gen_swz(16 * tp + lw, 4 + gw));
+          float4_t r = {0.f, 0.f, 0.f, 0.f};
+          r = mfma16x16x32(a0, f0, r);
+          r = mfma16x16x32(a1, f1, r);
+          *reinterpret_cast<float4_t*>(wown + 16 * tp + 4 * gw) = r;
+          // (four tiles in flight: with all reads ahead of all products B = 32,
+          // L = 256 takes 264 us)
+          if (tp % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      fetch(pkh, rg.c_lo);
+      stage_barrier();  // every wave holds its K fragments
+      if (lane < 16) wown[kGenWin] = -0.0f;
+      for (int w0 = rg.c_lo; w0 <= rg.c_hi; w0 += kGenWin) {  // uniform
+        put();
         stage_barrier();
-        products(rk, 0, q0, q1);
-        wave_lds_sync();
+        if (w0 + kGenWin <= rg.c_hi) fetch(pkh, w0 + kGenWin);
+        else fetch(pqh, rg.p_lo);
+        wide_products(q0, q1);
+        stage_barrier();  // every wave is done with the window
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[kb][j] += own[min((uint32_t)(c_of(cp[kb][j]) - w0), (uint32_t)kBiasCols)];
-        stage_barrier();
+          for (int j = 0; j < 4; ++j) acc[kb][j] += wown[min((uint32_t)(c_of(cp[kb][j]) - w0), (uint32_t)kGenWin)];
       }
-      for (int w0 = rg.p_lo; w0 <= rg.p_hi; w0 += kBiasCols) {  // uniform
-        issue_window(pqh, rq, w0);
-        wait_vmcnt<0>();
-        stage_barrier();
-        products(rq, 0, kp0, kp1);
+      for (int w0 = rg.p_lo; w0 <= rg.p_hi; w0 += kGenWin) {  // uniform
+        put();
+        stage_barrier();  // (and every wave is past the last window's gather)
+        if (w0 + kGenWin <= rg.p_hi) fetch(pqh, w0 + kGenWin);
+        wide_products(kp0, kp1);
         stage_barrier();
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             acc[kb][j] +=
-                tab[(16 * kb + 4 * g + j) * kBiasStride + min((uint32_t)(p_of(cp[kb][j]) - w0), (uint32_t)kBiasCols)];
-        stage_barrier();
+                wtab[(16 * kb + 4 * gw + j) * kWideStride + min((uint32_t)(p_of(cp[kb][j]) - w0), (uint32_t)kGenWin)];
       }
+      // (waited for here on every path: else the compiler waits for them, and
+      // for whatever was issued since, in the next block's narrow path)
+#pragma unroll
+      for (int i = 0; i < kGenWin / 32; ++i) asm volatile("" : "+v"(x[i]));
     }
     stage_barrier();  // P2C rows visible; every wave is done with both windows and the K rows
     const Range now = rg;

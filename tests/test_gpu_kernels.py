@@ -753,6 +753,31 @@ def test_general_index_kernels_any_length(L, P, H, B, relative):
     assert np.max(np.abs(got - want)) <= 2e-3  # one fp16 rounding of values below 4
 
 
+@pytest.mark.parametrize("L", [320, 333, 512])
+def test_fused_attention_wide_and_narrow_tiles_in_turn(L):
+    """Relative-position indices with whole 64 x 64 tiles of arbitrary ones
+    among them: a row of tiles goes from one table window to several and back,
+    in every order, through the same buffers."""
+    B, H, P = 2, 3, 512
+    r = np.random.default_rng(2500 + L)
+    q, k, v = (r.standard_normal((B, H, L, 64)).astype(np.float16) for _ in range(3))
+    pkh, pqh = (r.standard_normal((H, P, 64)).astype(np.float16) for _ in range(2))
+    idx = np.clip(O.relative_bucket(np.arange(L)[:, None] - np.arange(L)[None, :]) + 256, 0, P - 1).astype(np.int32)
+    c2p = np.broadcast_to(idx, (H, L, L)).copy()
+    p2c = np.broadcast_to(idx.T, (H, L, L)).copy()
+    tile = np.arange(L) // 64
+    wide = r.random((H, tile[-1] + 1, tile[-1] + 1)) < 0.5  # [h, query tile, key tile]
+    at = wide[:, tile][:, :, tile]
+    c2p[at] = r.integers(0, P, size=int(at.sum()))
+    at = (wide & (r.random(wide.shape) < 0.7))[:, tile][:, :, tile].transpose(0, 2, 1)  # some in c2p alone
+    p2c[at] = r.integers(0, P, size=int(at.sum()))
+    key_mask = np.where(r.random((B, L)) < 0.1, -65504.0, 0.0).astype(np.float16)
+    args = (q, k, v, pkh, pqh, c2p, p2c, key_mask)
+    want = O.fused_attention_kernel(*args, O.scale_f32(64))
+    got = host(fk().fused_attention(*map(dev, args), O.scale_f32(64), B, H, L, 64, P))
+    assert np.max(np.abs(got - want)) <= 2e-3  # one fp16 rounding of values below 4
+
+
 @pytest.mark.parametrize("relative", [True, False])
 @pytest.mark.parametrize("L,H,B", [(256, 16, 5), (252, 16, 5), (254, 16, 5), (253, 16, 5), (512, 3, 3)])
 def test_relative_bias_several_batch_rows(L, H, B, relative):
