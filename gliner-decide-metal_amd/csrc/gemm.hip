@@ -968,10 +968,10 @@ int launch_lds_tile_gelu320(const half_t* A, const half_t* W, const half_t* bias
   return GD_OK;
 }
 
-template <bool GATHER>
+template <int BM, bool GATHER>
 int launch_tile(const half_t* A, const half_t* W, const half_t* bias, half_t* C, int M, int N, int K, int64_t lda,
                 int64_t ldc, const int32_t* a_rows, int a_row_count, int epi, hipStream_t stream) {
-  constexpr int BM = 128, BN = 128;
+  constexpr int BN = 128;
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = N / BN;
   const dim3 grid(tiles_m * tiles_n), block(kThreads);
@@ -1303,8 +1303,8 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
   // operands take the register-staged kernel (same accumulation order).
   const int64_t a_last = (a_rows ? a_row_count : m) - 1;
   if (a_last * lda + K >= (int64_t{1} << 31) || (int64_t)N * K >= (int64_t{1} << 31)) {
-    if (a_rows) return launch_tile<true>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
-    return launch_tile<false>(A, Wt, Bv, Cm, M, N, K, lda, ldc, nullptr, 0, epilogue_kind, stream);
+    if (a_rows) return launch_tile<128, true>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
+    return launch_tile<128, false>(A, Wt, Bv, Cm, M, N, K, lda, ldc, nullptr, 0, epilogue_kind, stream);
   }
   const int64_t cus = gemm_cu_count();
   const bool gelu = epilogue_kind == GD_EPI_BIAS_GELU;
@@ -1315,7 +1315,8 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
     // 15.7 on 64 x 64 tiles, QKV at 64 and 128 rows 4.4 and 5.2 against 6.4;
     // in a second round they lose: QKV at 300 rows 9.7 against 6.9).
     if (K % kSkBK == 0) {
-      if (M <= 32) return launch_skinny<2, 1, 8>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
+      if (M <= 32 && (!a_rows || N / 16 <= cus))
+        return launch_skinny<2, 1, 8>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
       if ((int64_t)((M + 31) / 32) * (N / 32) <= cus)
         return launch_skinny<2, 2, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
       if ((int64_t)((M + 63) / 64) * (N / 32) <= cus)
@@ -1324,11 +1325,20 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
     return kNoTile;
   };
   if (a_rows) {
+    // A K of up to three steps gives the DMA stages nothing to run ahead of: the
+    // register-staged tiles start sooner (K = 64 at 1 to 700 rows 3.9 to 4.6 us
+    // against 4.4 to 5.0, K = 192 4.9 to 5.6 against 5.2 to 5.8; from 1,024 rows
+    // on the DMA tiles are as fast or faster).
+    if (K <= 192 && M < 1024)
+      return launch_tile<64, true>(A, Wt, Bv, Cm, M, N, K, lda, ldc, a_rows, (int)a_row_count, epilogue_kind, stream);
     const GatheredRows rows{a_rows, (int)a_row_count};
     const int st = with_rows(rows);
     if (st != kNoTile) return st;
-    // Gathered rows (marker rows, at most a few thousand): the cheaper of two tiles.
-    if (cheapest_tile(M, N, K, gelu, cus, 2) == 0)
+    // Gathered rows (marker rows, at most a few thousand): the cheaper of two
+    // tiles, 64 x 64 for at most four rounds of them (beyond, the model's share
+    // is too small: 1,500 x 4096 x 2048, six rounds, 47 us where it has 40 for
+    // either tile).
+    if ((int64_t)((M + 63) / 64) * (N / 64) <= 4 * cus && cheapest_tile(M, N, K, gelu, cus, 2) == 0)
       return launch_lds_tile<64, 64, 2, 64, 4, 4>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream, rows);
     return launch_lds_tile<128, 128, 2, 64, 2, 8>(A, Wt, Bv, Cm, M, N, K, lda, ldc, epilogue_kind, stream, rows);
   }

@@ -152,13 +152,15 @@ def test_linear_gelu_table_under_the_last_k_steps(m, k):
 
 
 @pytest.mark.parametrize("n,k,epilogue", [(1024, 4096, "bias"), (3072, 1024, "bias"), (4096, 1024, "gelu"),
-                                          (2048, 1024, "relu"), (384, 192, "bias")])
+                                          (2048, 1024, "relu"), (384, 192, "bias"), (2048, 64, "relu"),
+                                          (8192, 256, "gelu")])
 def test_linear_few_rows_and_gathered_rows(n, k, epilogue):
     """Every row of a product has the bits that the 8,192-row product gives
     it, at the row counts where the skinny tiles change (32 rows, one round of
     32-row and of 64-row tiles, K = 192 without them), and where the rows are
     gathered (any order, repeats; indices outside the operand read the nearest
-    row, as the clamp states)."""
+    row, as the clamp states), at a K for the register-staged tiles and at a
+    width that leaves the 32 x 16 tiles too."""
     g = torch.Generator(device="cuda")
     g.manual_seed(n + k)
     x = torch.randn((8192, k), generator=g, device="cuda").half()
@@ -173,6 +175,26 @@ def test_linear_few_rows_and_gathered_rows(n, k, epilogue):
         assert torch.equal(fk().linear(x, w, b, epilogue, rows=rows), full[rows.long()]), m
     rows = torch.tensor([-5, 0, 8191, 9000] * 20, dtype=torch.int32, device="cuda")
     assert torch.equal(fk().linear(x, w, b, epilogue, rows=rows), full[rows.long().clamp(0, 8191)])
+
+
+def test_linear_operand_past_2_31_elements():
+    """A of more than 2^31 elements takes the register-staged tiles with 64-bit
+    addresses: rows on either side of the bound, plain and gathered, have the
+    bits of the small products."""
+    k, n, m = 1024, 128, 2 ** 21 + 1
+    g = torch.Generator(device="cuda")
+    g.manual_seed(31)
+    x = torch.empty((m, k), dtype=torch.float16, device="cuda").normal_(generator=g)
+    w = (0.02 * torch.randn((n, k), generator=g, device="cuda")).half()
+    b = torch.randn((n,), generator=g, device="cuda").half()
+    full = fk().linear(x, w, b, "bias")
+    for lo in (0, 2 ** 20 - 150, m - 300):
+        assert torch.equal(fk().linear(x[lo:lo + 300].contiguous(), w, b, "bias"), full[lo:lo + 300]), lo
+    ends = torch.tensor([m - 1, 0, m - 2, 1, 2 ** 20, m - 1], dtype=torch.int32, device="cuda")
+    rows = torch.cat([ends, torch.randint(0, m, (150,), generator=g, device="cuda", dtype=torch.int32)])
+    for epilogue in ("none", "bias", "relu", "gelu"):
+        want = fk().linear(x[rows.long()], w, b, epilogue)
+        assert torch.equal(fk().linear(x, w, b, epilogue, rows=rows), want), epilogue
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 128, 64), (65, 256, 128), (300, 1024, 1024), (1000, 384, 192),
