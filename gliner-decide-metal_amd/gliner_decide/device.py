@@ -25,12 +25,18 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return t.data_ptr()
 
 
+# The current stream's handle alone, where this torch has such a call (it is not
+# part of its public interface): a torch.cuda.Stream object costs more than the
+# rest of a small call's arguments.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(stream: torch.cuda.Stream | None = None) -> int:
-    if stream is not None:
-        return stream.cuda_stream
-    # The handle alone: a torch.cuda.Stream object costs more than the rest of
-    # a small call's arguments.
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if stream is None:
+        if _raw_stream is not None:
+            return _raw_stream(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
+    return stream.cuda_stream
 
 
 def as_f16(t: torch.Tensor, name: str) -> torch.Tensor:

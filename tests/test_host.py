@@ -188,3 +188,22 @@ def test_decode_multi_label_extreme_logits():
     assert p0.labels == ["b"] and p0.probabilities[0] == 0.0 and p0.probabilities[2] == 0.0
     p1 = decode(logits, 1, tasks)[0]
     assert p1.probabilities == [0.0, 0.0, 0.0] and p1.labels == ["a"]  # first of equal maxima
+
+
+def test_stream_handle_falls_back_to_the_public_stream(monkeypatch):
+    """The raw handle call is not part of torch's public interface: without it
+    the current stream's object gives the handle, as an explicit stream does."""
+    from gliner_decide import device
+
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+    monkeypatch.setattr(device, "_raw_stream", None)
+    monkeypatch.setattr(device.torch.cuda, "current_stream", lambda: Stream(17))
+    assert device.stream_handle() == 17
+    assert device.stream_handle(Stream(5)) == 5
+    monkeypatch.setattr(device, "_raw_stream", lambda index: 100 + index)
+    monkeypatch.setattr(device.torch.cuda, "current_device", lambda: 3)
+    assert device.stream_handle() == 103
+    assert device.stream_handle(Stream(5)) == 5
