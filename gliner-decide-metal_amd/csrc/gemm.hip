@@ -22,7 +22,8 @@
 //     on a few hundred): tiles of 32 x 16 to 64 x 32, a wave for each 16 x 16
 //     on v_mfma_f32_16x16x16_f16, four or eight 128-deep stages;
 //   * gemm_nt_kernel, register-staged (global -> registers -> LDS, one K step
-//     ahead): operands that exceed 32-bit element offsets.
+//     ahead): operands that exceed 32-bit element offsets, gathered rows of a
+//     short K.
 // Rows may be gathered through an index list (the classifier's marker rows):
 // the DMA kernels look each row up once, where they form its address.
 // Every kernel accumulates an element over the same 16-wide K slices in the
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_nt_lds_kernel(const half_t* __re
     // Two-stage tiles that read the full GELU table bring it under the last K steps: those
     // have nothing left to fetch, and each part of the table goes into the
     // buffer that has just become free (4,096 columns on 32,768, 8,192 and 4,896
-    // rows 307 -> 296, 85.7 -> 83.8 and 49.2 -> 47.8 us against a table brought
+    // rows 294 -> 285, 77.4 -> 74.9 and 49.3 -> 48.1 us against a table brought
     // after the loop).  The bias epilogues keep the loop below: without a table
     // the tail gained nothing, and K = 4096 lost 5% to it.
     auto issue_table = [&](auto b) {
@@ -1006,7 +1007,7 @@ int launch_tile(const half_t* A, const half_t* W, const half_t* bias, half_t* C,
 // v_mfma_f32_16x16x16_f16 chain and a workgroup MB x NB of them, small enough
 // that the product is spread over the chip, with NST 128-deep stages of A and W
 // in flight (64 to 96 KiB).  FFN-down (K = 4096) at 64, 256 and 300 rows takes
-// 7.8, 8.1 and 10.2 us where the 64 x 64 tiles take 15.4 to 15.7; above a chain's
+// 8.2, 8.5 and 10.5 us where the 64 x 64 tiles take 15.6 to 15.8; above a chain's
 // 4.3 us it is bound by what a CU draws from its L2.  The 16 x 16 x 16 MFMA
 // sums the same 16 products per K slice as the 32 x 32 x 16 form, bit for bit
 // (gd_diag_mfma_forms runs both on the device; a GPU test compares them over
@@ -1067,7 +1068,7 @@ __global__ __launch_bounds__(64 * MB * NB) void gemm_skinny_kernel(const half_t*
   const int wm = wave % MB, wn = wave / MB;  // 16 rows, 16 columns
   const int g = lane >> 4, r = lane & 15;
 
-  // This lane's 16-byte pieces: block j of the wave (stage block 6 w + j)
+  // This lane's 16-byte pieces: block j of the wave (stage block kSkLoads w + j)
   // holds rows 4 blk .. 4 blk + 3, lane l row 4 blk + l / 16 at physical
   // chunk l % 16, which is logical chunk (l % 16) ^ (row & 15).  Rows past M
   // repeat row M - 1 (never stored).  Offsets in elements, 32-bit.
@@ -1307,10 +1308,15 @@ int launch_linear(const void* a, const void* w, const void* bias, void* c, int64
   const bool gelu = epilogue_kind == GD_EPI_BIAS_GELU;
   auto with_rows = [&](auto rows) -> int {
     // Few rows: skinny tiles, 32 rows on 16 columns up to 32 rows, else the
-    // smaller of 32 x 32 and 64 x 32 that fits one round of workgroups (FFN-down
-    // at 64, 256, 300 and 512 rows 7.8, 8.1, 10.2 and 11.5 us against 15.4 to
-    // 15.7 on 64 x 64 tiles, QKV at 64 and 128 rows 4.4 and 5.2 against 6.4;
-    // in a second round they lose: QKV at 300 rows 9.7 against 6.9).
+    // smaller of 32 x 32 and 64 x 32 that gives each CU at most one workgroup
+    // (FFN-down at 64, 256, 300 and 512 rows 8.2, 8.5, 10.5 and 11.9 us against
+    // 15.6 to 16.1 on 64 x 64 tiles, QKV at 64 and 128 rows 4.6 and 5.5 against
+    // 6.4 to 6.5).  Two 32 x 32 workgroups fit a CU, but where 64 x 32 gives each
+    // one they are slower (QKV at 128 rows 5.8 against 5.5, FFN-down at 300 10.9
+    // against 10.5); past that only QKV at 136 to 160 rows gains by them (5.9
+    // against 6.6).  Up to 32 rows the 32 x 32 tiles take 4.3 to 4.8 us at K = 1024
+    // where the 32 x 16 take 4.5 to 4.95, and 8.1 where those take 8.0 at K = 4096.
+    // Gathered rows take the latter only where each CU has at most one.
     if (K % kSkBK == 0) {
       if (M <= 32 && (!a_rows || N / 16 <= cus))
         return launch_skinny<2, 1, 8>(A, Wt, Bv, Cm, M, N, K, lda, ldc, rows, epilogue_kind, stream);
