@@ -204,6 +204,6 @@ def test_stream_handle_falls_back_to_the_public_stream(monkeypatch):
     assert device.stream_handle() == 17
     assert device.stream_handle(Stream(5)) == 5
     monkeypatch.setattr(device, "_raw_stream", lambda index: 100 + index)
-    monkeypatch.setattr(device.torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(device, "_current_device", lambda: 3)
     assert device.stream_handle() == 103
     assert device.stream_handle(Stream(5)) == 5
