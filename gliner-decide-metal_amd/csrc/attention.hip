@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64) void fused_attention_general_kernel(
 // H = 16, L = 512: 18.1 us so, 14.5 through LDS; L = 256: 6.4 and 6.0).
 //
 // Several batch rows are bound by the batch row's chain (MFMA, table, gather,
-// barrier, store) with two waves per SIMD (250 VGPRs).  B = 32, H = 16, L =
+// barrier, store) with two waves per SIMD (254 VGPRs).  B = 32, H = 16, L =
 // 256: 36 us against 71 us of a kernel that read indices and table rows for
 // every batch row and ran 64-row windows of either table, a gather per window;
 // at 5 TB/s its 111 MB take 22 us.  Random indices (the whole table for every
@@ -183,7 +183,7 @@ constexpr int bias_waves(bool multi) { return multi ? 2 : 3; }
 // pieces (every row starts aligned to one); from 4 on the c2p indices and the
 // mask of four consecutive keys are one aligned load.  MULTI: the workgroup
 // walks several batch rows.  With one there is nothing to keep: P2C takes the
-// C2P rows' place, and kBiasOneWaves workgroups share a CU.
+// C2P rows' place, and three workgroups share a CU.
 template <int W, bool MULTI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bias_waves(MULTI), bias_waves(MULTI)))) void relative_bias_mfma_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ pos_key,
